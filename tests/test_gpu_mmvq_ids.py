@@ -48,6 +48,25 @@ def test_small_formats(t, n_in, n_out, ncols):
 
 
 @pytest.mark.parametrize("t", ALL)
+@pytest.mark.parametrize("shift", [4, 8, 12])
+def test_mmvq_matrix_on_a_4_byte_boundary(t, shift):
+    """The products read a row's fields as the aligned words around them: a matrix that starts 4, 8 or 12 bytes behind a
+    16-byte boundary, with rows of an odd number of blocks (every block start that the format's size allows), gives the
+    bits of the same matrix on a 256-byte boundary and the exact integer sums."""
+    n_in, n_out = 768, 21
+    print(f"4-byte boundary t={t} shift={shift}", flush=True)
+    w = weights(t, n_out, n_in, 300 + t)
+    xq = O.quantize_q8_1(np.random.default_rng(t).normal(0, 1, (2, n_in)).astype(np.float32))
+    buf = torch.zeros(w.size + shift + 16, dtype=torch.uint8, device="cuda")
+    buf[shift:shift + w.size] = dev(w.ravel())
+    got = host(ops.iq_mmvq(t, buf[shift:], dev(xq), n_in, n_out, 2))
+    assert np.array_equal(got, host(ops.iq_mmvq(t, dev(w), dev(xq), n_in, n_out, 2)))
+    s, q = ops.subblock_sums(t, buf[shift:], n_in, n_out, dev(xq), 2)
+    es, eq = O.subblock_sums(t, w, n_in, n_out, xq, 2)
+    assert (host(s) == es).all() and (host(q) == eq).all()
+
+
+@pytest.mark.parametrize("t", ALL)
 @pytest.mark.parametrize("x_every", [1, 3])
 def test_mmvq_ids(t, x_every):
     n_in, n_out, n_mat, count = 512, 80, 6, 11

@@ -53,12 +53,12 @@ __global__ void __launch_bounds__(kThreads) swiglu_entries_kernel(const float* _
 // acc[c] = row . x[c] for c < n, the row's LPR lanes each taking units l, l + LPR, ...; reduced over the LPR lanes
 template <int T, int LPR, int NC>
 __device__ __forceinline__ void row_dots(const uint8_t* __restrict__ row, const tsx_block_q8_1* const (&xs)[NC], int n,
-                                         int nu, int l, float (&acc)[NC]) {
+                                         int nu, int l, const LdsTab<T>& tab, float (&acc)[NC]) {
 #pragma unroll
     for (int c = 0; c < NC; ++c) acc[c] = 0.f;
     for (int u = l; u < nu; u += LPR) {
         Unit w;
-        unit_load<T>(row, u, w, grid_const());
+        unit_load_global<T>(row, u, w, tab);
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             if (c < n) {
@@ -81,6 +81,9 @@ __global__ void __launch_bounds__(kThreads) expert_gu_kernel(const uint64_t* __r
                                                              const int32_t* __restrict__ ent_tok,
                                                              const tsx_block_q8_1* __restrict__ xq, tsx_expert_layout L,
                                                              float* __restrict__ gate, float* __restrict__ up) {
+    __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
+    const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
+    if constexpr (lds_tab_words<T>() > 0) __syncthreads();
     constexpr int RPW = kWave / LPR;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
@@ -102,7 +105,7 @@ __global__ void __launch_bounds__(kThreads) expert_gu_kernel(const uint64_t* __r
 #pragma unroll
             for (int c = 0; c < kNC; ++c) xs[c] = xq + (int64_t) ent_tok[e + min(c, n - 1)] * nu;
             float acc[kNC];
-            row_dots<T, LPR, kNC>(wr, xs, n, nu, l, acc);
+            row_dots<T, LPR, kNC>(wr, xs, n, nu, l, tab, acc);
             if (l == 0)
                 for (int c = 0; c < n; ++c) dst[(int64_t) (e + c) * FF + r] = acc[c];
         }
@@ -117,6 +120,9 @@ __global__ void __launch_bounds__(kThreads) expert_down_kernel(const uint64_t* _
                                                                const int32_t* __restrict__ ent_dst,
                                                                const tsx_block_q8_1* __restrict__ hq, tsx_expert_layout L,
                                                                float* __restrict__ out) {
+    __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
+    const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
+    if constexpr (lds_tab_words<T>() > 0) __syncthreads();
     constexpr int RPW = kWave / LPR;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
@@ -135,7 +141,7 @@ __global__ void __launch_bounds__(kThreads) expert_down_kernel(const uint64_t* _
 #pragma unroll
             for (int c = 0; c < kNC; ++c) xs[c] = hq + (int64_t) (e + min(c, n - 1)) * nu;
             float acc[kNC];
-            row_dots<T, LPR, kNC>(wr, xs, n, nu, l, acc);
+            row_dots<T, LPR, kNC>(wr, xs, n, nu, l, tab, acc);
             if (l == 0)
                 for (int c = 0; c < n; ++c) out[(int64_t) ent_dst[e + c] * N + r] = acc[c];
         }
@@ -147,6 +153,9 @@ template <int T, int LPR>
 __global__ void __launch_bounds__(kThreads) mmvq_kernel(const uint8_t* __restrict__ w, uint64_t row_bytes,
                                                         const tsx_block_q8_1* __restrict__ x, float* __restrict__ y,
                                                         int n_in, int n_out, int ncols) {
+    __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
+    const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
+    if constexpr (lds_tab_words<T>() > 0) __syncthreads();
     constexpr int RPW = kWave / LPR;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
@@ -160,7 +169,7 @@ __global__ void __launch_bounds__(kThreads) mmvq_kernel(const uint8_t* __restric
 #pragma unroll
         for (int c = 0; c < kNC; ++c) xs[c] = x + (int64_t) (c0 + min(c, n - 1)) * nu;
         float acc[kNC];
-        row_dots<T, LPR, kNC>(wr, xs, n, nu, l, acc);
+        row_dots<T, LPR, kNC>(wr, xs, n, nu, l, tab, acc);
         if (l == 0)
             for (int c = 0; c < n; ++c) y[(int64_t) (c0 + c) * n_out + r] = acc[c];
     }
@@ -200,6 +209,9 @@ struct SlotsSource {
 };
 template <int T, int LPR, typename Src>
 __global__ void __launch_bounds__(kThreads) mmvq_many_kernel(Src src, uint64_t row_bytes, int n_in, int n_out) {
+    __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
+    const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
+    if constexpr (lds_tab_words<T>() > 0) __syncthreads();
     constexpr int RPW = kWave / LPR;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
@@ -214,7 +226,7 @@ __global__ void __launch_bounds__(kThreads) mmvq_many_kernel(Src src, uint64_t r
     }
     const tsx_block_q8_1* xs[1] = {xj};
     float acc[1];
-    row_dots<T, LPR, 1>(w + (uint64_t) r * row_bytes, xs, 1, n_in / 32, l, acc);
+    row_dots<T, LPR, 1>(w + (uint64_t) r * row_bytes, xs, 1, n_in / 32, l, tab, acc);
     if (l == 0) yj[r] = acc[0];
 }
 
@@ -229,7 +241,7 @@ __global__ void __launch_bounds__(kThreads) subblock_sums_kernel(const uint8_t* 
     const int64_t r = i / nu;
     const int u = (int) (i % nu);
     Unit wu;
-    unit_load<T>(w + (uint64_t) r * row_bytes, u, wu, grid_const());
+    unit_load_global<T>(w + (uint64_t) r * row_bytes, u, wu, grid_const());
     for (int64_t c = 0; c < ncols; ++c) {
         Act a;
         act_load(x + c * nu + u, a);

@@ -150,6 +150,32 @@ template <int T> __device__ __forceinline__ SignEntry tab_sign(const RepTab<T>& 
     return SignEntry{(uint32_t) v, (uint32_t) (v >> 32)};
 }
 
+// T's codebook and sign entries once in LDS, for kernels whose blocks are too short-lived for the copies above (the
+// constant tables are global memory: a unit's twelve lookups are gathers there)
+template <int T> constexpr int lds_tab_words() { return rep_grid_entries<T>() + 2 * rep_sign_entries<T>(); }
+template <int T>
+struct LdsTab {
+    lds_ptr<const uint32_t> grid, sign;
+};
+// every thread of the block stores its share; a barrier has to follow before the first read
+template <int T, int NT>
+__device__ __forceinline__ LdsTab<T> lds_tab_fill(uint32_t* lds) {
+    constexpr int NG = rep_grid_entries<T>(), N = lds_tab_words<T>();
+    const uint32_t* g = T == TSX_IQ3_XXS ? kGrid.xxs : kGrid.s;
+    const uint32_t* sg = (const uint32_t*) (T == TSX_IQ3_XXS ? kGrid.xxs_sign : kGrid.s_sign);
+#pragma unroll
+    for (int k = 0; k < (N + NT - 1) / NT; ++k) {
+        const int i = (int) threadIdx.x + NT * k;
+        if (i < N) ((lds_ptr<uint32_t>) lds)[i] = i < NG ? g[i] : sg[i - NG];
+    }
+    return LdsTab<T>{(lds_ptr<const uint32_t>) lds, (lds_ptr<const uint32_t>) lds + NG};
+}
+template <int T> __device__ __forceinline__ uint32_t tab_grid(const LdsTab<T>& r, uint32_t i) { return r.grid[i]; }
+template <int T> __device__ __forceinline__ SignEntry tab_sign(const LdsTab<T>& r, uint32_t i) {
+    const uint64_t v = ((lds_ptr<const uint64_t>) r.sign)[i];
+    return SignEntry{(uint32_t) v, (uint32_t) (v >> 32)};
+}
+
 // ------------------------------------------------------------------ scalar helpers
 __device__ __forceinline__ float h2f(uint16_t h) { return (float) __builtin_bit_cast(_Float16, h); }
 __device__ __forceinline__ uint16_t f2h(float f) { return __builtin_bit_cast(uint16_t, (_Float16) f); }
@@ -253,48 +279,132 @@ __device__ __forceinline__ void unit_load_q80(const uint8_t* row, int u, Unit& o
     o.b = 0.f;
 }
 
-// Q4_0: the 4-bit codes as they are (0..15); the -8 offset is applied with the activation block's sum
-__device__ __forceinline__ void unit_load_q40(const uint8_t* row, int u, Unit& o) {
-    const uint8_t* blk = row + u * 18;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const uint32_t q = ld32a2(blk + 2 + 4 * k);
-        o.w[k] = (int) (q & 0x0F0F0F0Fu);              // values 4k .. 4k + 3
-        o.w[4 + k] = (int) ((q >> 4) & 0x0F0F0F0Fu);   // values 16 + 4k ..
-    }
-    o.a = h2f((uint16_t) ld16(blk));
-    o.b = 0.f;
-}
-
-// Q6_K unit u = half u / 4, quarter u % 4 of the block: value l (0..31) of the quarter is the low (quarters 0, 1)
-// or high (2, 3) nibble of ql[64 half + 32 (quarter % 2) + l] with bits 2 quarter .. 2 quarter + 1 of
-// qh[32 half + l] above it, minus 32; the scale of values 0-15 is scales[8 half + 2 quarter], of 16-31 the next.
-// The codes stay unsigned (0..63): the -32 is applied with each half's activation sum
-__device__ __forceinline__ void unit_load_q6k(const uint8_t* row, int u, Unit& o) {
-    const uint8_t* blk = row + (u >> 3) * 210;
-    const int j = u & 7, half = j >> 2, qt = j & 3;
-    const uint8_t* ql = blk + 64 * half + 32 * (qt & 1);
-    const uint8_t* qh = blk + 128 + 32 * half;
-    const int lsh = 4 * (qt >> 1), hsh = 2 * qt;
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-        o.w[k] = (int) (((ld32a2(ql + 4 * k) >> lsh) & 0x0F0F0F0Fu) | (((ld32a2(qh + 4 * k) >> hsh) & 0x03030303u) << 4));
-    const int8_t* sc = (const int8_t*) (blk + 192 + 8 * half + 2 * qt);
-    o.k0 = sc[0];
-    o.k1 = sc[1];
-    o.a = h2f((uint16_t) ld16(blk + 208));
-    o.b = 0.f;
-}
-
-// unit u of a row of format T; g: where the codebooks are read (GridRef or RepTab<T>)
+// unit u of a row of an expert format T in LDS; g: where the codebooks are read (RepTab<T>)
 template <int T, typename Tab>
 __device__ __forceinline__ void unit_load(const uint8_t* row, int u, Unit& o, const Tab& g) {
     if constexpr (T == TSX_IQ3_XXS) unit_load_iq3xxs(row, u, o, g);
     else if constexpr (T == TSX_IQ3_S) unit_load_iq3s(row, u, o, g);
     else if constexpr (T == TSX_Q4_K) unit_load_q4k(row, u, o);
-    else if constexpr (T == TSX_Q4_0) unit_load_q40(row, u, o);
-    else if constexpr (T == TSX_Q6_K) unit_load_q6k(row, u, o);
     else unit_load_q80(row, u, o);
+}
+
+// ------------------------------------------------------------------ unit decode from global memory
+// unit_load reads a unit's fields as 16-bit words, which an LDS slab serves well and global memory does not: a Q4_K unit
+// is 22 load instructions of two bytes a lane.  Here the aligned 4-byte words around the fields are read in 16-byte
+// pieces and shifted into place: three load instructions for a Q4_K unit, three for Q8_0, eight for Q6_K.  Rows start on
+// 2-byte boundaries at least, as GGUF blocks of an even size do behind a 4-byte aligned matrix.  Only words that hold
+// bytes of the field are read.  Four dense products of 2048 x 6144 by four columns with their quantize launches: Q6_K
+// 55 -> 41 us, Q8_0 54 -> 40, Q4_K 46 -> 36; IQ3_S, its codebook in LDS (LdsTab), 51 -> 39.
+typedef int v4i_a4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef int v2i_a4 __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ uint32_t gld16(uintptr_t a) { return *(gbl_ptr<const uint16_t>) a; }
+__device__ __forceinline__ uint32_t gld8(uintptr_t a) { return *(gbl_ptr<const uint8_t>) a; }
+// 4 N bytes at a (2-byte aligned) as N words, N = 1, 2, 4 or 8.  shift (0 or 16) tells whether the bytes straddle words
+template <int N> __device__ __forceinline__ void gld_words(uintptr_t a, uint32_t (&w)[N]) {
+    const uintptr_t b = a & ~(uintptr_t) 3;
+    const uint32_t sh = (uint32_t) (a & 2) * 8;
+    uint32_t r[N + 1];
+    if constexpr (N >= 4) {
+#pragma unroll
+        for (int k = 0; k < N / 4; ++k) {
+            const v4i_a4 v = *(gbl_ptr<const v4i_a4>) (b + 16 * k);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r[4 * k + i] = (uint32_t) v[i];
+        }
+    } else if constexpr (N == 2) {
+        const v2i_a4 v = *(gbl_ptr<const v2i_a4>) b;
+        r[0] = (uint32_t) v.x;
+        r[1] = (uint32_t) v.y;
+    } else {
+        r[0] = *(gbl_ptr<const uint32_t>) b;
+    }
+    // the word after: read where the bytes straddle, else the last one again
+    r[N] = *(gbl_ptr<const uint32_t>) (b + 4 * (N - 1) + 2 * (a & 2));
+#pragma unroll
+    for (int k = 0; k < N; ++k) w[k] = __builtin_amdgcn_alignbit(r[k + 1], r[k], sh);
+}
+template <int T, typename Tab>
+__device__ __forceinline__ void unit_load_global(const uint8_t* row, int u, Unit& o, const Tab& g) {
+    const uintptr_t blk = (uintptr_t) row + (uintptr_t) (u / Fmt<T>::upb * Fmt<T>::bytes);
+    const int j = u % Fmt<T>::upb;
+    o.b = 0.f;
+    if constexpr (T == TSX_IQ3_XXS) {
+        uint32_t q[2], aux[1];
+        const float d = h2f((uint16_t) gld16(blk));
+        gld_words<2>(blk + 2 + 8 * j, q);
+        gld_words<1>(blk + 66 + 4 * j, aux);
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            const SignEntry sg = tab_sign<TSX_IQ3_XXS>(g, (aux[0] >> (7 * l)) & 127u);
+            const uint32_t i0 = (q[l >> 1] >> (16 * (l & 1))) & 255u, i1 = (q[l >> 1] >> (16 * (l & 1) + 8)) & 255u;
+            o.w[2 * l] = (int) apply_signs(tab_grid<TSX_IQ3_XXS>(g, i0), sg.mask_lo);
+            o.w[2 * l + 1] = (int) apply_signs(tab_grid<TSX_IQ3_XXS>(g, i1), sg.mask_hi);
+        }
+        o.a = d * 0.25f * (float) (2 * (int) (aux[0] >> 28) + 1);
+    } else if constexpr (T == TSX_IQ3_S) {
+        uint32_t q[2], sb[1];
+        const float d = h2f((uint16_t) gld16(blk));
+        gld_words<2>(blk + 2 + 8 * j, q);
+        gld_words<1>(blk + 74 + 4 * j, sb);
+        const uint32_t qh = gld8(blk + 66 + j);
+        const uint32_t sc = (gld8(blk + 106 + (j >> 1)) >> (4 * (j & 1))) & 15u;
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            const SignEntry sg = tab_sign<TSX_IQ3_S>(g, (sb[0] >> (8 * l)) & 255u);
+            const int k0 = 2 * l, k1 = 2 * l + 1;
+            const uint32_t i0 = ((q[l >> 1] >> (8 * (k0 & 3))) & 255u) | (((qh >> k0) & 1u) << 8);
+            const uint32_t i1 = ((q[l >> 1] >> (8 * (k1 & 3))) & 255u) | (((qh >> k1) & 1u) << 8);
+            o.w[k0] = (int) apply_signs(tab_grid<TSX_IQ3_S>(g, i0), sg.mask_lo);
+            o.w[k1] = (int) apply_signs(tab_grid<TSX_IQ3_S>(g, i1), sg.mask_hi);
+        }
+        o.a = d * (float) (2 * (int) sc + 1);
+    } else if constexpr (T == TSX_Q4_K) {
+        uint32_t h[4], q[8];
+        gld_words<4>(blk, h);
+        gld_words<8>(blk + 16 + 32 * (j >> 1), q);
+        const int sh = 4 * (j & 1);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) o.w[k] = (int) ((q[k] >> sh) & 0x0F0F0F0Fu);
+        // scale and min byte of sub-block j: 0-3 the low 6 bits of bytes 0-3 and 4-7 of the 12, 4-7 the nibbles of bytes
+        // 8-11 with the top 2 bits of bytes 0-3 and 4-7 above them
+        const uint32_t lo = 0u - (uint32_t) (j < 4);
+        const uint32_t SC = (h[1] & 0x3F3F3F3Fu & lo) | (((h[3] & 0x0F0F0F0Fu) | ((h[1] >> 2) & 0x30303030u)) & ~lo);
+        const uint32_t M = (h[2] & 0x3F3F3F3Fu & lo) | ((((h[3] >> 4) & 0x0F0F0F0Fu) | ((h[2] >> 2) & 0x30303030u)) & ~lo);
+        o.a = h2f((uint16_t) h[0]) * (float) ((SC >> (8 * (j & 3))) & 255u);
+        o.b = h2f((uint16_t) (h[0] >> 16)) * (float) ((M >> (8 * (j & 3))) & 255u);
+    } else if constexpr (T == TSX_Q4_0) {
+        // the 4-bit codes as they are (0..15); the -8 offset is applied with the activation block's sum
+        uint32_t q[4];
+        gld_words<4>(blk + 2, q);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {  // values 4 k .. 4 k + 3, and 16 + 4 k ..
+            o.w[k] = (int) (q[k] & 0x0F0F0F0Fu);
+            o.w[4 + k] = (int) ((q[k] >> 4) & 0x0F0F0F0Fu);
+        }
+        o.a = h2f((uint16_t) gld16(blk));
+    } else if constexpr (T == TSX_Q6_K) {
+        // half j / 4, quarter j % 4 of the block: value l (0..31) of the quarter is the low (quarters 0, 1) or high (2,
+        // 3) nibble of ql[64 half + 32 (quarter % 2) + l] with bits 2 quarter .. 2 quarter + 1 of qh[32 half + l] above
+        // it, minus 32; the scale of values 0-15 is scales[8 half + 2 quarter], of 16-31 the next.  The codes stay
+        // unsigned (0..63): the -32 is applied with each half's activation sum
+        const int half = j >> 2, qt = j & 3, lsh = 4 * (qt >> 1), hsh = 2 * qt;
+        uint32_t ql[8], qh[8];
+        gld_words<8>(blk + 64 * half + 32 * (qt & 1), ql);
+        gld_words<8>(blk + 128 + 32 * half, qh);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            o.w[k] = (int) (((ql[k] >> lsh) & 0x0F0F0F0Fu) | (((qh[k] >> hsh) & 0x03030303u) << 4));
+        const uint32_t sc = gld16(blk + 192 + 8 * half + 2 * qt);  // two int8 scales
+        o.k0 = (int) (int8_t) sc;
+        o.k1 = (int) (int8_t) (sc >> 8);
+        o.a = h2f((uint16_t) gld16(blk + 208));
+    } else {
+        uint32_t q[8];
+        gld_words<8>(blk + 2, q);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) o.w[k] = (int) q[k];
+        o.a = h2f((uint16_t) gld16(blk));
+    }
 }
 
 // one Q8_1 activation block: d, the sum field s and the 32 codes as 8 words
@@ -303,11 +413,17 @@ struct Act {
     float d, s;
 };
 __device__ __forceinline__ void act_load(const tsx_block_q8_1* x, Act& a) {
-    const uint32_t* p = (const uint32_t*) x;
-    a.d = h2f((uint16_t) (p[0] & 0xFFFFu));
-    a.s = h2f((uint16_t) (p[0] >> 16));
+    // 36 bytes on a 4-byte boundary of global memory
+    const uintptr_t p = (uintptr_t) x;
+    const uint32_t ds = *(gbl_ptr<const uint32_t>) p;
+    const v4i_a4 q0 = *(gbl_ptr<const v4i_a4>) (p + 4), q1 = *(gbl_ptr<const v4i_a4>) (p + 20);
+    a.d = h2f((uint16_t) (ds & 0xFFFFu));
+    a.s = h2f((uint16_t) (ds >> 16));
 #pragma unroll
-    for (int k = 0; k < 8; ++k) a.q[k] = (int) p[1 + k];
+    for (int k = 0; k < 4; ++k) {
+        a.q[k] = q0[k];
+        a.q[4 + k] = q1[k];
+    }
 }
 
 // the unit's contribution to a row . activation dot product; *S (and *M) the exact integer sums

@@ -149,6 +149,9 @@ __global__ void __launch_bounds__(kThreads) mmq_rows_kernel(const uint8_t* __res
                                                             const int32_t* __restrict__ bounds,
                                                             const int32_t* __restrict__ ids, float* __restrict__ dst,
                                                             int64_t ld_dst) {
+    __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
+    const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
+    if constexpr (lds_tab_words<T>() > 0) __syncthreads();
     constexpr int RPW = kWave / LPR;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
@@ -163,7 +166,7 @@ __global__ void __launch_bounds__(kThreads) mmq_rows_kernel(const uint8_t* __res
         float acc[kNC] = {0.f, 0.f, 0.f, 0.f};
         for (int u = l; u < nu; u += LPR) {
             Unit wu;
-            unit_load<T>(wr, u, wu, grid_const());
+            unit_load_global<T>(wr, u, wu, tab);
 #pragma unroll
             for (int c = 0; c < kNC; ++c) {
                 if (c < n) {
