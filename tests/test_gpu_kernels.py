@@ -115,6 +115,18 @@ def test_mmvq(t, n_in, n_out, ncols):
     np.testing.assert_allclose(got, exp, rtol=1e-5, atol=1e-5 * np.abs(exp).max())
 
 
+@pytest.mark.parametrize("n_in,n_out", [(2048, 4095), (2048, 4097), (2048, 8195), (256, 32771)])
+def test_mmvq_rows_per_wave(n_in, n_out):
+    """The row counts at which a wave takes one, two and four rows of each lane group, and remainders of them: every row
+    once, against the oracle."""
+    rng = np.random.default_rng(n_out)
+    w = np.tile(ops.quantize_weights(Q4_K, rng.normal(0, 0.02, (61, n_in)).astype(np.float32)), (n_out // 61 + 1, 1))[:n_out]
+    xq = O.quantize_q8_1(rng.normal(0, 1, (5, n_in)).astype(np.float32))
+    got = host(ops.iq_mmvq(Q4_K, dev(w), dev(xq), n_in, n_out, 5))
+    exp = np.tile(O.mmvq_q8_1(Q4_K, w[:61], n_in, 61, xq, 5), (1, n_out // 61 + 1))[:, :n_out]
+    np.testing.assert_allclose(got, exp, rtol=1e-5, atol=1e-5 * np.abs(exp).max())
+
+
 @pytest.mark.parametrize("E,k,T", [(256, 8, 1), (256, 8, 4), (128, 8, 512), (64, 4, 7), (512, 16, 3)])
 def test_router_topk(E, k, T):
     rng = np.random.default_rng(E + k + T)

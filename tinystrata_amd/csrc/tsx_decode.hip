@@ -5,8 +5,8 @@
 // 1489-1515, down rows 1407-1465, q8_1 1467-1487, mmvq 716-740); src/kernels/cuda/native_mmvq.cu:154-185.
 //
 // Layout on the chip: a weight row is split over LPR lanes of a wave64 (LPR = the row's 32-value units rounded
-// up to a power of two, at most 64), so a wave reads 64/LPR rows at once; each lane decodes a unit once and
-// applies it to every entry of the group (up to NC at a time), then the row's lanes reduce.  A block is 4 waves;
+// up to a power of two, at most 64), so a wave reads 64/LPR rows at once, R of them a lane group; each lane decodes a
+// unit once and applies it to every entry of the group (up to NC at a time), then the row's lanes reduce.  A block is 4 waves;
 // gate and up rows of the same index lie in the same block row so the whole expert is read once per group.
 #include "tsx_common.hpp"
 #include "tsx_device.hpp"
@@ -50,31 +50,58 @@ __global__ void __launch_bounds__(kThreads) swiglu_entries_kernel(const float* _
 }
 
 // ------------------------------------------------------------------ row dots
-// acc[c] = row . x[c] for c < n, the row's LPR lanes each taking units l, l + LPR, ...; reduced over the LPR lanes
-template <int T, int LPR, int NC>
-__device__ __forceinline__ void row_dots(const uint8_t* __restrict__ row, const tsx_block_q8_1* const (&xs)[NC], int n,
-                                         int nu, int l, const LdsTab<T>& tab, float (&acc)[NC]) {
+// acc[j][c] = rows[j] . x[c] for c < n, the R rows' LPR lanes each taking units l, l + LPR, ...; reduced over the LPR
+// lanes.  A unit's activations (36 bytes a column, against 18 of Q4_K weights) are read once for the R rows
+template <int T, int LPR, int NC, int R>
+__device__ __forceinline__ void row_dots(const uint8_t* const (&rows)[R], const tsx_block_q8_1* const (&xs)[NC], int n,
+                                         int nu, int l, const LdsTab<T>& tab, float (&acc)[R][NC]) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] = 0.f;
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[j][c] = 0.f;
     for (int u = l; u < nu; u += LPR) {
-        Unit w;
-        unit_load_global<T>(row, u, w, tab);
+        Unit w[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) unit_load_global<T>(rows[j], u, w[j], tab);
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             if (c < n) {
                 Act a;
                 act_load(xs[c] + u, a);
-                int S, M;
-                acc[c] += unit_dot<T>(w, a, S, M);
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    int S, M;
+                    acc[j][c] += unit_dot<T>(w[j], a, S, M);
+                }
             }
         }
     }
 #pragma unroll
-    for (int c = 0; c < NC; ++c) acc[c] = group_sum<LPR>(acc[c]);
+    for (int j = 0; j < R; ++j)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[j][c] = lanes_sum<LPR>(acc[j][c]);  // (every lane of the wave calls)
+}
+// Rows per wave and pass: R of each LPR-lane group, as many of 4, 2 and 1 as leave kRowsPerWaveMin waves, eight a CU.
+// Several rows share a unit's activation loads and a block's chain of table reads; with fewer waves than that more waves
+// hide more of the chain than the shared loads save (2048 x 6144 Q6_K by 4 columns and its quantize: 10.4 us with one
+// row a wave, 9.4 with two, 10.7 with four).  With the sums over lanes by DPP instead of LDS permutes: wide experts
+// (4096 x 1536 Q4_K, 8 groups) 56 -> 49 us a layer, in IQ3 64 -> 49
+constexpr int64_t kRowsPerWaveMin = 2048;
+inline int rows_per_lane_group(int64_t rows, int lpr) {
+    const int64_t waves = rows / (kWave / lpr);
+    return waves >= 4 * kRowsPerWaveMin ? 4 : waves >= 2 * kRowsPerWaveMin ? 2 : 1;
+}
+template <typename F>
+int with_rows(int r, F&& f) {
+    switch (r) {
+        case 4: return f(std::integral_constant<int, 4>{});
+        case 2: return f(std::integral_constant<int, 2>{});
+        default: return f(std::integral_constant<int, 1>{});
+    }
 }
 
 // gate and up rows of every group: gate[e][r], up[e][r] for the group's entries e
-template <int T, int LPR>
+template <int T, int LPR, int R>
 __global__ void __launch_bounds__(kThreads) expert_gu_kernel(const uint64_t* __restrict__ grp_ptr,
                                                              const int32_t* __restrict__ grp_start,
                                                              const int32_t* __restrict__ n_groups,
@@ -88,32 +115,43 @@ __global__ void __launch_bounds__(kThreads) expert_gu_kernel(const uint64_t* __r
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
     const int FF = (int) L.n_ff, nu = (int) (L.n_embd / 32);
-    const int row = (blockIdx.x * (kThreads / kWave) + wave) * RPW + slot;
-    const bool valid = row < 2 * FF;
-    const bool is_up = valid && row >= FF;
-    const int r = is_up ? row - FF : (valid ? row : 0);
-    const uint64_t off = (is_up ? L.up_off : 0) + (uint64_t) r * L.gu_row;
-    float* dst = is_up ? up : gate;
+    const int row0 = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
+    uint64_t off[R];
+    float* dst[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) {  // a row past the last repeats the last and stores nothing
+        const int row = min(row0 + RPW * j, 2 * FF - 1);
+        const bool is_up = row >= FF;
+        const int r = is_up ? row - FF : row;
+        off[j] = (is_up ? L.up_off : 0) + (uint64_t) r * L.gu_row;
+        dst[j] = (is_up ? up : gate) + r;
+    }
     const int ng = *n_groups;
     for (int g = blockIdx.y; g < ng; g += gridDim.y) {
-        if (!valid) continue;
-        const uint8_t* wr = (const uint8_t*) grp_ptr[g] + off;
+        const uint8_t* wr[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) wr[j] = (const uint8_t*) grp_ptr[g] + off[j];
         const int e0 = grp_start[g], e1 = grp_start[g + 1];
         for (int e = e0; e < e1; e += kNC) {
             const int n = min(kNC, e1 - e);
             const tsx_block_q8_1* xs[kNC];
 #pragma unroll
             for (int c = 0; c < kNC; ++c) xs[c] = xq + (int64_t) ent_tok[e + min(c, n - 1)] * nu;
-            float acc[kNC];
-            row_dots<T, LPR, kNC>(wr, xs, n, nu, l, tab, acc);
+            float acc[R][kNC];
+            row_dots<T, LPR, kNC, R>(wr, xs, n, nu, l, tab, acc);
             if (l == 0)
-                for (int c = 0; c < n; ++c) dst[(int64_t) (e + c) * FF + r] = acc[c];
+#pragma unroll
+                for (int j = 0; j < R; ++j)
+                    if (row0 + RPW * j < 2 * FF)
+#pragma unroll
+                        for (int c = 0; c < kNC; ++c)
+                            if (c < n) dst[j][(int64_t) (e + c) * FF] = acc[j][c];
         }
     }
 }
 
 // down rows: out[ent_dst[e]][r] = down_r . hq[e]
-template <int T, int LPR>
+template <int T, int LPR, int R>
 __global__ void __launch_bounds__(kThreads) expert_down_kernel(const uint64_t* __restrict__ grp_ptr,
                                                                const int32_t* __restrict__ grp_start,
                                                                const int32_t* __restrict__ n_groups,
@@ -127,29 +165,34 @@ __global__ void __launch_bounds__(kThreads) expert_down_kernel(const uint64_t* _
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
     const int N = (int) L.n_embd, nu = (int) (L.n_ff / 32);
-    const int r = (blockIdx.x * (kThreads / kWave) + wave) * RPW + slot;
-    const bool valid = r < N;
-    const uint64_t off = L.down_off + (uint64_t) (valid ? r : 0) * L.d_row;
+    const int r0 = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
     const int ng = *n_groups;
     for (int g = blockIdx.y; g < ng; g += gridDim.y) {
-        if (!valid) continue;
-        const uint8_t* wr = (const uint8_t*) grp_ptr[g] + off;
+        const uint8_t* wr[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+            wr[j] = (const uint8_t*) grp_ptr[g] + L.down_off + (uint64_t) min(r0 + RPW * j, N - 1) * L.d_row;
         const int e0 = grp_start[g], e1 = grp_start[g + 1];
         for (int e = e0; e < e1; e += kNC) {
             const int n = min(kNC, e1 - e);
             const tsx_block_q8_1* xs[kNC];
 #pragma unroll
             for (int c = 0; c < kNC; ++c) xs[c] = hq + (int64_t) (e + min(c, n - 1)) * nu;
-            float acc[kNC];
-            row_dots<T, LPR, kNC>(wr, xs, n, nu, l, tab, acc);
+            float acc[R][kNC];
+            row_dots<T, LPR, kNC, R>(wr, xs, n, nu, l, tab, acc);
             if (l == 0)
-                for (int c = 0; c < n; ++c) out[(int64_t) ent_dst[e + c] * N + r] = acc[c];
+#pragma unroll
+                for (int j = 0; j < R; ++j)
+                    if (r0 + RPW * j < N)
+#pragma unroll
+                        for (int c = 0; c < kNC; ++c)
+                            if (c < n) out[(int64_t) ent_dst[e + c] * N + r0 + RPW * j] = acc[j][c];
         }
     }
 }
 
 // y[c][r] = W[r] . x[c], ncols <= 8 columns
-template <int T, int LPR>
+template <int T, int LPR, int R>
 __global__ void __launch_bounds__(kThreads) mmvq_kernel(const uint8_t* __restrict__ w, uint64_t row_bytes,
                                                         const tsx_block_q8_1* __restrict__ x, float* __restrict__ y,
                                                         int n_in, int n_out, int ncols) {
@@ -160,18 +203,24 @@ __global__ void __launch_bounds__(kThreads) mmvq_kernel(const uint8_t* __restric
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
     const int nu = n_in / 32;
-    const int r = (blockIdx.x * (kThreads / kWave) + wave) * RPW + slot;
-    if (r >= n_out) return;  // whole LPR groups leave together
-    const uint8_t* wr = w + (uint64_t) r * row_bytes;
+    const int r0 = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
+    const uint8_t* wr[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) wr[j] = w + (uint64_t) min(r0 + RPW * j, n_out - 1) * row_bytes;
     for (int c0 = 0; c0 < ncols; c0 += kNC) {
         const int n = min(kNC, ncols - c0);
         const tsx_block_q8_1* xs[kNC];
 #pragma unroll
         for (int c = 0; c < kNC; ++c) xs[c] = x + (int64_t) (c0 + min(c, n - 1)) * nu;
-        float acc[kNC];
-        row_dots<T, LPR, kNC>(wr, xs, n, nu, l, tab, acc);
+        float acc[R][kNC];
+        row_dots<T, LPR, kNC, R>(wr, xs, n, nu, l, tab, acc);
         if (l == 0)
-            for (int c = 0; c < n; ++c) y[(int64_t) (c0 + c) * n_out + r] = acc[c];
+#pragma unroll
+            for (int j = 0; j < R; ++j)
+                if (r0 + RPW * j < n_out)
+#pragma unroll
+                    for (int c = 0; c < kNC; ++c)
+                        if (c < n) y[(int64_t) (c0 + c) * n_out + r0 + RPW * j] = acc[j][c];
     }
 }
 
@@ -207,7 +256,7 @@ struct SlotsSource {
         return true;
     }
 };
-template <int T, int LPR, typename Src>
+template <int T, int LPR, int R, typename Src>
 __global__ void __launch_bounds__(kThreads) mmvq_many_kernel(Src src, uint64_t row_bytes, int n_in, int n_out) {
     __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
     const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
@@ -215,19 +264,22 @@ __global__ void __launch_bounds__(kThreads) mmvq_many_kernel(Src src, uint64_t r
     constexpr int RPW = kWave / LPR;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
-    const int r = (blockIdx.x * (kThreads / kWave) + wave) * RPW + slot;
-    if (r >= n_out) return;  // whole LPR groups leave together
+    const int r0 = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
     const uint8_t* w = nullptr;
     const tsx_block_q8_1* xj = nullptr;
     float* yj = nullptr;
-    if (!src.at((int) blockIdx.y, w, xj, yj)) {  // an id outside the table: the matrix's outputs are zero
-        if (l == 0) yj[r] = 0.f;
-        return;
+    float acc[R][1] = {};
+    if (src.at((int) blockIdx.y, w, xj, yj)) {  // else an id outside the table: the matrix's outputs are zero
+        const tsx_block_q8_1* xs[1] = {xj};
+        const uint8_t* wr[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) wr[j] = w + (uint64_t) min(r0 + RPW * j, n_out - 1) * row_bytes;
+        row_dots<T, LPR, 1, R>(wr, xs, 1, n_in / 32, l, tab, acc);
     }
-    const tsx_block_q8_1* xs[1] = {xj};
-    float acc[1];
-    row_dots<T, LPR, 1>(w + (uint64_t) r * row_bytes, xs, 1, n_in / 32, l, tab, acc);
-    if (l == 0) yj[r] = acc[0];
+    if (l == 0)
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+            if (r0 + RPW * j < n_out) yj[r0 + RPW * j] = acc[j][0];
 }
 
 // the integer contract, one thread per (row, unit)
@@ -303,10 +355,12 @@ int launch_many(const char* what, int type, const Src& src, int count, int n_in,
     const int lpr = lanes_per_row(n_in / 32), rows = (kThreads / kWave) * (kWave / lpr);
     return with_mmvq_type(type, [&](auto T) {
         return with_lpr(lpr, [&](auto LPR) {
-            const dim3 grid(blocks_for(n_out, rows), (unsigned) count);
-            mmvq_many_kernel<decltype(T)::value, decltype(LPR)::value, Src>
-                <<<grid, kThreads, 0, (hipStream_t) stream>>>(src, rb, n_in, n_out);
-            return launch_status(what);
+            return with_rows(rows_per_lane_group((int64_t) n_out * count, lpr), [&](auto R) {
+                const dim3 grid(blocks_for(n_out, rows * decltype(R)::value), (unsigned) count);
+                mmvq_many_kernel<decltype(T)::value, decltype(LPR)::value, decltype(R)::value, Src>
+                    <<<grid, kThreads, 0, (hipStream_t) stream>>>(src, rb, n_in, n_out);
+                return launch_status(what);
+            });
         });
     });
 }
@@ -364,10 +418,12 @@ TSX_API int tsx_moe_expert_grouped(const tsx_expert_layout* Lp, const uint64_t* 
     const int rows_gu = (kThreads / kWave) * (kWave / lpr_gu), rows_d = (kThreads / kWave) * (kWave / lpr_d);
     int rc = with_type(L.gu_type, [&](auto T) {
         return with_lpr(lpr_gu, [&](auto LPR) {
-            const dim3 grid(blocks_for(2 * L.n_ff, rows_gu), (unsigned) gy);
-            expert_gu_kernel<decltype(T)::value, decltype(LPR)::value>
-                <<<grid, kThreads, 0, s>>>(grp_ptr, grp_start, n_groups, ent_tok, X, L, gate, up);
-            return launch_status("tsx_moe_expert_grouped/gate-up");
+            return with_rows(rows_per_lane_group(2 * L.n_ff * gy, lpr_gu), [&](auto R) {
+                const dim3 grid(blocks_for(2 * L.n_ff, rows_gu * decltype(R)::value), (unsigned) gy);
+                expert_gu_kernel<decltype(T)::value, decltype(LPR)::value, decltype(R)::value>
+                    <<<grid, kThreads, 0, s>>>(grp_ptr, grp_start, n_groups, ent_tok, X, L, gate, up);
+                return launch_status("tsx_moe_expert_grouped/gate-up");
+            });
         });
     });
     if (rc != TSX_OK) return rc;
@@ -379,10 +435,12 @@ TSX_API int tsx_moe_expert_grouped(const tsx_expert_layout* Lp, const uint64_t* 
     }
     return with_type(L.d_type, [&](auto T) {
         return with_lpr(lpr_d, [&](auto LPR) {
-            const dim3 grid(blocks_for(L.n_embd, rows_d), (unsigned) gy);
-            expert_down_kernel<decltype(T)::value, decltype(LPR)::value>
-                <<<grid, kThreads, 0, s>>>(grp_ptr, grp_start, n_groups, ent_dst, hq, L, out);
-            return launch_status("tsx_moe_expert_grouped/down");
+            return with_rows(rows_per_lane_group(L.n_embd * gy, lpr_d), [&](auto R) {
+                const dim3 grid(blocks_for(L.n_embd, rows_d * decltype(R)::value), (unsigned) gy);
+                expert_down_kernel<decltype(T)::value, decltype(LPR)::value, decltype(R)::value>
+                    <<<grid, kThreads, 0, s>>>(grp_ptr, grp_start, n_groups, ent_dst, hq, L, out);
+                return launch_status("tsx_moe_expert_grouped/down");
+            });
         });
     });
 }
@@ -400,9 +458,12 @@ TSX_API int tsx_moe_mmvq(int type, const void* w, const void* x_q8_1, float* y, 
     const int lpr = lanes_per_row(n_in / 32), rows = (kThreads / kWave) * (kWave / lpr);
     return with_mmvq_type(type, [&](auto T) {
         return with_lpr(lpr, [&](auto LPR) {
-            mmvq_kernel<decltype(T)::value, decltype(LPR)::value><<<blocks_for(n_out, rows), kThreads, 0, (hipStream_t) stream>>>(
-                (const uint8_t*) w, rb, (const tsx_block_q8_1*) x_q8_1, y, n_in, n_out, ncols);
-            return launch_status("tsx_moe_mmvq");
+            return with_rows(rows_per_lane_group(n_out, lpr), [&](auto R) {
+                mmvq_kernel<decltype(T)::value, decltype(LPR)::value, decltype(R)::value>
+                    <<<blocks_for(n_out, rows * decltype(R)::value), kThreads, 0, (hipStream_t) stream>>>(
+                        (const uint8_t*) w, rb, (const tsx_block_q8_1*) x_q8_1, y, n_in, n_out, ncols);
+                return launch_status("tsx_moe_mmvq");
+            });
         });
     });
 }
