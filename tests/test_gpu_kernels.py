@@ -247,11 +247,12 @@ def test_mmq_quantize_route_matches_the_two_calls(rows, E, k):
 
 @pytest.mark.parametrize("shared,prow,n", [(False, False, 2048), (True, True, 2048), (True, False, 4096),
                                            (False, True, 96)])
-def test_combine_norm(shared, prow, n):
+@pytest.mark.parametrize("pad,k", [(0, 8), (0, 3), (1, 8)])   # rows 16-byte aligned (four columns per thread), and not
+def test_combine_norm(shared, prow, n, pad, k):
     """tsx_moe_combine_norm: x is tsx_moe_combine's x bit for bit; h the closed-form norm of it (within float32
     rounding); hq the Q8_1 image of h byte for byte."""
     rng = np.random.default_rng(n + shared)
-    T, k, eps = 37, 8, 1e-5
+    T, eps = 37, 1e-5
     parts = rng.normal(0, 1, (T * k, n)).astype(np.float32)
     wts = rng.random((T, k)).astype(np.float32)
     x = rng.normal(0, 1, (T, n)).astype(np.float32)
@@ -264,7 +265,7 @@ def test_combine_norm(shared, prow, n):
     x_plain = dev(x)
     ops.moe_combine(x_plain, pd, wd, k, prow=pr, shared=sh, sgate=sg)
     xd = dev(x)
-    h = torch.full((T, n), float("nan"), device="cuda")
+    h = torch.full((T * n + pad,), float("nan"), device="cuda")[pad:].view(T, n)
     hq = torch.zeros((T, n // 32 * 36), dtype=torch.uint8, device="cuda")
     ops.moe_combine_norm(xd, pd, wd, k, dev(wn), eps, h, hq, prow=pr, shared=sh, sgate=sg)
     xv, hv = host(xd), host(h)
