@@ -427,6 +427,74 @@ def test_mmq_run_tile_classes(t):
     np.testing.assert_allclose(got, exp, rtol=1e-5, atol=1e-5 * np.abs(exp).max())
 
 
+FEW_COUNTS = [0, 1, 2, 3, 5, 16, 17, 33, 0, 8, 4, 1]  # at most eight rows per expert on average
+
+
+@pytest.mark.parametrize("t", [IQ3_XXS, IQ3_S, Q4_K])
+@pytest.mark.parametrize("w_cols,w_rows,pad", [(256, 64, 0), (512, 448, 1), (768, 320, 0), (2048, 128, 0), (1280, 192, 3)])
+def test_mmq_run_few_rows(t, w_cols, w_rows, pad):
+    """The few-rows form: experts of 0 to 33 rows (tiles of 1 to 16 rows, whose windows hold 16 chunks down to one), odd
+    and even chunk counts (IQ3 rows on 2- and 4-byte boundaries), one and two passes with a part of a pass left over,
+    output rows on and off 16-byte boundaries; activation units whose scales lie a factor of 1e8 apart within a chunk;
+    against the oracle's per-row dot on the same Q8_1 codes."""
+    rng = np.random.default_rng(t + w_cols + w_rows)
+    n, total = len(FEW_COUNTS), sum(FEW_COUNTS)
+    assert total <= 8 * n
+    bounds = np.concatenate([[0], np.cumsum(FEW_COUNTS)]).astype(np.int32)
+    W = [ops.quantize_weights(t, rng.normal(0, 0.02, (w_rows, w_cols)).astype(np.float32)) for _ in range(n)]
+    rb = W[0].shape[1]
+    eb = (w_rows * rb + 255) // 256 * 256
+    blob = np.zeros(n * eb, np.uint8)
+    for i, m in enumerate(W):
+        blob[i * eb: i * eb + m.size] = m.ravel()
+    x = rng.normal(0, 1, (total, w_cols)).astype(np.float32)
+    x[1::3, 32:64] *= 1e4
+    x[1::3, 64:96] *= 1e-4
+    x[2::5, :256] = 0.0                                # a chunk of zero scales
+    ids = rng.permutation(total).astype(np.int32)
+    xq = ops.mmq_quantize(dev(x), None, t, w_cols, w_cols, total)
+    ld = w_rows + pad
+    dst = torch.full((total, ld), float("nan"), device="cuda")
+    ops.mmq_run(dev(blob), t, w_rows, w_cols, eb, n, xq, dev(bounds), dev(ids), total, dst, ld)
+    got = host(dst)
+    assert np.isnan(got[:, w_rows:]).all()
+    xb = O.quantize_q8_1(x)
+    exp = np.zeros((total, w_rows), np.float64)
+    for i in range(n):
+        r0, r1 = bounds[i], bounds[i + 1]
+        if r1 > r0:
+            exp[ids[r0:r1]] = O.mmvq_q8_1(t, W[i], w_cols, w_rows, xb[r0:r1], r1 - r0)
+    assert np.isfinite(got[:, :w_rows]).all()
+    scale = np.abs(exp).max(axis=1, keepdims=True)     # per token: the tokens' magnitudes are a factor of 1e4 apart
+    assert (np.abs(got[:, :w_rows] - exp) <= 1e-5 * np.abs(exp) + 1e-5 * scale).all()
+
+
+@pytest.mark.parametrize("t", [IQ3_XXS, IQ3_S, Q4_K])
+@pytest.mark.parametrize("N,FF,counts", [(512, 128, FEW_COUNTS), (2048, 384, FEW_COUNTS), (768, 256, [64]), (256, 128, [1])])
+def test_mmq_gate_up_swiglu_few_rows(t, N, FF, counts):
+    """The few-rows form of the fused gate/up launch against the call sequence on the GPU: the same planes byte for
+    byte."""
+    rng = np.random.default_rng(t + N + FF)
+    n, total = len(counts), sum(counts)
+    bounds = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    W = ops.quantize_weights(t, rng.normal(0, 0.05, (n * 2 * FF, N)).astype(np.float32)).reshape(n, -1)
+    eb = (W.shape[1] + 255) // 256 * 256
+    blob = np.zeros((n, eb), np.uint8)
+    blob[:, :W.shape[1]] = W
+    x = rng.normal(0, 1, (40, N)).astype(np.float32)
+    x[:, rng.choice(N, N // 50, replace=False)] *= 20.0
+    xids = rng.integers(0, 40, total).astype(np.int32)
+    blob_d, bounds_d = dev(blob.ravel()), dev(bounds)
+    xq_rows = ops.mmq_quantize(dev(x), dev(xids), t, N, N, total)
+    gu = torch.empty((total, 2 * FF), device="cuda")
+    ops.mmq_run(blob_d, t, 2 * FF, N, eb, n, xq_rows, bounds_d, None, total, gu, 2 * FF)
+    ref = ops.mmq_quantize(ops.mmq_swiglu(gu, total, FF), None, t, FF, FF, total)
+    xq_tok = ops.mmq_quantize(dev(x), None, t, N, N, 40)
+    got = ops.mmq_gate_up_swiglu(blob_d, t, FF, N, eb, n, xq_tok, 40, dev(xids), bounds_d, total)
+    for a, b in zip(_planes(got, total, FF), _planes(ref, total, FF)):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+
+
 def _planes(buf, rows: int, cols: int):
     """The Q8_1 planes of tsx_moe_mmq_q8_bytes: codes, block scales and code sums of the first `rows` rows."""
     b = host(buf)

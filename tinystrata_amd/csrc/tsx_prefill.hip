@@ -1016,6 +1016,422 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     else run(std::integral_constant<int, (kBN >= 128 ? 8 : 4)>{});
 }
 
+// ------------------------------------------------------------------ grouped product, few rows per expert
+// Up to kSTok token rows a tile: a serving batch or a short prompt, where an expert's weights serve one or a few rows.
+// Block (weight-row tile bx, token tile): 32 kSWaves rows of one expert's matrix a pass, `passes` passes; each wave owns
+// 32 rows (two 16-row MFMA tiles) and every token of the tile.
+//
+// The product runs on v_mfma_f32_16x16x32_f16 with exact operands and no scale left per 32-value unit:
+//   A = the unit's weight codes times the integer part of its scale (IQ3_XXS: grid * sign * (2 ls + 1) <= 1922; IQ3_S:
+//       <= 15 * 31; Q4_K: q * sc <= 945), an integer that fp16 holds;
+//   B = the activations with their scale, code * dx, as the sum of two fp16 numbers.  dx is an fp16 value, so the
+//       product has at most 18 bits: hi is the product rounded to a multiple of 2^e (dx in [2^e, 2^(e+1)): 8 bits), lo
+//       the rest (10 bits), both exact once dx has been multiplied by the power of two that puts the largest of the
+//       token's scales in the 256-value chunk in [16, 32) (exact while the chunk's scales lie within 2^18 of each
+//       other; a smaller one loses bits below 2^-40 of the chunk's largest product).
+// The sums over hi are integers of a common power of two that rarely need more than 24 bits, and lo has accumulators of
+// its own, so a chunk's sum is nearly exact in fp32; times the row's float scale and the token's power of two it is
+// added to the row's total (Q4_K's min term is a K = 8 product on the fp32 matrix cores).  Relative error against 64
+// bits over 768 columns: IQ3 4.4e-8 (the 128-token tiles above: 1.8e-7), Q4_K 1.5e-7 (3.2e-7).
+//
+// Because no scale is left outside, the units of a chunk may meet in one MFMA: lane group g takes units 2 g and 2 g + 1
+// of the chunk, eight values a step.  A lane then reads its weights as 16 (Q4_K: 32) consecutive bytes from global
+// memory straight into registers, a chunk ahead, and the waves of a block share nothing but the activations: those lie
+// in LDS in the order the MFMA reads them, [step][hi, lo][lane group][token] 16 bytes, packed for the tile's rows, so
+// that a window of 16 / rows chunks fits (with one or two rows a whole row of 2048) and most tiles meet one barrier in
+// all.  What bounds it is vector issue (about 23 instructions for 512 weights, the codebook's share) beside HBM, and a
+// block's fixed chain (tile search, row index, codes: ~5 us); against the 128-token tiles, whose blocks of eight waves
+// alone on a CU wait for each chunk's loads at a barrier, a batch of 32 tokens (256 experts top-8, IQ3) takes 57 us
+// instead of 116 for gate/up and 38 instead of 66 for down; 200 tokens: two layers 291 -> 187 us each.  A codebook with
+// the signs applied (32 KB, one lookup instead of two) measured the same: it saves vector work but halves the blocks
+// that share a CU.
+constexpr int kSTok = 16;
+constexpr int kSWaves = 4;  // per block
+constexpr int kSWindow = 64 * 64 * kSWaves;  // LDS bytes of a window: a half unit of 16 codes per thread
+// waves per SIMD that the registers are held to: four for the codebook formats (128 registers, no spills), three for
+// Q4_K, whose raw rows are wider (at four it spills: a batch of 32, gate/up and down 126 -> 117 us a layer with three)
+template <int T> constexpr int small_wpe() { return T == TSX_Q4_K ? 3 : 4; }
+template <int T> constexpr int small_grid() { return T == TSX_IQ3_XXS ? 256 : T == TSX_IQ3_S ? 512 : 0; }
+// the codebook (four fp16 magnitudes an entry) and the sixteen masks of four sign bits
+template <int T> constexpr int small_tab_bytes() { return small_grid<T>() > 0 ? 8 * small_grid<T>() + 128 : 0; }
+template <int T> struct SmallLds {
+    static constexpr int TAB = 0, B = TAB + small_tab_bytes<T>();
+    static constexpr int DW = B + kSWindow;                // float [kSWaves][32]: the rows' scales of the chunk
+    static constexpr int EX = DW + kSWaves * 128;          // int [chunk of the window][token]: the exponents
+    static constexpr int DR = EX + kSWindow / 1024 * 4;    // int [kSTok]: the token's output row
+    static constexpr int SCAN = DR + kSTok * 4;
+    static constexpr int DM = SCAN + (kSWaves + 2) * 8;    // Q4_K: float [chunk][unit][token]: min-term factors
+    static constexpr int BYTES = DM + (T == TSX_Q4_K ? kSWindow / 1024 * 8 * 4 : 0);
+};
+
+typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+
+// a lane's weights of one 16-row tile and chunk as loaded (aligned words around its bytes)
+template <int T> struct MmqRaw;
+template <> struct MmqRaw<TSX_IQ3_XXS> { v4i q; int q4; v2i a; int a2; uint16_t d; };
+template <> struct MmqRaw<TSX_IQ3_S> { v4i q; int q4; v2i a; int a2; uint16_t qh, d; uint8_t sc; };
+template <> struct MmqRaw<TSX_Q4_K> { v4i h, q[2]; };
+// the row's block of the chunk lies at base + o (base 4-byte aligned and the same in every lane); lane group g takes
+// units 2 g and 2 g + 1
+template <int T> __device__ __forceinline__ void raw_load(MmqRaw<T>& R, gbl_ptr<const uint8_t> base, uint32_t o, int g) {
+    if constexpr (T == TSX_Q4_K) {
+        R.h = *(gbl_ptr<const v4i>) (base + o);
+        R.q[0] = *(gbl_ptr<const v4i>) (base + (o + 16 + 32 * g));
+        R.q[1] = *(gbl_ptr<const v4i>) (base + (o + 32 + 32 * g));
+    } else {
+        // the words that hold the lane's bytes: they start on a 2-byte boundary, and where that is a 4-byte one the
+        // extra word is the last one again
+        const uint32_t q = (o + 2 + 16 * g) & ~3u, a = (o + (T == TSX_IQ3_XXS ? 66 : 74) + 8 * g) & ~3u;
+        const uint32_t odd = ((o + 2) & 2) * 2;  // 4 where the bytes straddle words
+        R.q = *(gbl_ptr<const v4i_a4>) (base + q);
+        R.q4 = *(gbl_ptr<const int>) (base + (q + 12 + odd));
+        R.a = *(gbl_ptr<const v2i_a4>) (base + a);
+        R.a2 = *(gbl_ptr<const int>) (base + (a + 4 + odd));
+        R.d = *(gbl_ptr<const uint16_t>) (base + o);
+        if constexpr (T == TSX_IQ3_S) {
+            R.qh = *(gbl_ptr<const uint16_t>) (base + (o + 66 + 2 * g));
+            R.sc = base[o + 106 + g];
+        }
+    }
+}
+// what a chunk's steps take besides R: the two units' sign words and fp16 scale pairs, the row's scale, Q4_K's mins
+template <int T> struct MmqScale {
+    uint32_t a[2], m[2];
+    float d, mn[2];
+};
+template <int T> __device__ __forceinline__ void raw_scales(const MmqRaw<T>& R, int sft, int g, MmqScale<T>& S) {
+    if constexpr (T == TSX_Q4_K) {
+        const uint32_t dd = (uint32_t) R.h[0];
+        S.d = h2f((uint16_t) dd);
+        // sub-blocks 2 g and 2 g + 1: scale and min bytes (sub-blocks 0-3: the low 6 bits of bytes 0-3 and 4-7; 4-7: the
+        // nibbles of bytes 8-11 with the top 2 bits of bytes 0-3 and 4-7 above them)
+        const uint32_t w0 = (uint32_t) R.h[1], w1 = (uint32_t) R.h[2], w2 = (uint32_t) R.h[3];
+        const uint32_t lo = 0u - (uint32_t) (g < 2);
+        const uint32_t SC = (w0 & 0x3F3F3F3Fu & lo) | (((w2 & 0x0F0F0F0Fu) | ((w0 >> 2) & 0x30303030u)) & ~lo);
+        const uint32_t M = (w1 & 0x3F3F3F3Fu & lo) | ((((w2 >> 4) & 0x0F0F0F0Fu) | ((w1 >> 2) & 0x30303030u)) & ~lo);
+        const int b0 = 16 * (g & 1);
+        const float dmin = -h2f((uint16_t) (dd >> 16));
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            S.m[k] = hpair((SC >> (b0 + 8 * k)) & 255u);
+            S.mn[k] = dmin * (float) ((M >> (b0 + 8 * k)) & 255u);
+        }
+    } else {
+        S.a[0] = __builtin_amdgcn_alignbit((uint32_t) R.a.y, (uint32_t) R.a.x, sft);
+        S.a[1] = __builtin_amdgcn_alignbit((uint32_t) R.a2, (uint32_t) R.a.y, sft);
+        const float d = h2f(R.d);
+        S.d = T == TSX_IQ3_XXS ? 0.25f * d : d;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if constexpr (T == TSX_IQ3_XXS) S.m[k] = hpair(2 * (S.a[k] >> 28) + 1);
+            else S.m[k] = hpair(2 * (((uint32_t) R.sc >> (4 * k)) & 15u) + 1);
+    }
+}
+// step s of the chunk (a constant once unrolled): values 8 (s % 4) .. + 7 of unit 2 g + s / 4, as the MFMA's A fragment
+template <int T> __device__ __forceinline__ v4i raw_frag(const MmqRaw<T>& R, const MmqScale<T>& S, int sft, int s,
+                                                         const uint8_t* tab) {
+    uint32_t f[4];
+    if constexpr (T == TSX_Q4_K) {
+        const uint32_t x0 = ((uint32_t) R.q[(s & 3) >> 1][2 * (s & 1)] >> (4 * (s >> 2))) & 0x0F0F0F0Fu;
+        const uint32_t x1 = ((uint32_t) R.q[(s & 3) >> 1][2 * (s & 1) + 1] >> (4 * (s >> 2))) & 0x0F0F0F0Fu;
+        const h2 sc = __builtin_bit_cast(h2, S.m[s >> 2]);
+        const h2 nsc = sc * (_Float16) -1024.0f;
+        nib_to_h(x0, sc, nsc, f[0], f[1]);
+        nib_to_h(x1, sc, nsc, f[2], f[3]);
+    } else {
+        const int k = s >> 1;
+        const uint32_t q = __builtin_amdgcn_alignbit(k == 3 ? (uint32_t) R.q4 : (uint32_t) R.q[(k + 1) & 3],
+                                                     (uint32_t) R.q[k], sft);
+        uint32_t a0 = (s & 1 ? q >> 13 : q << 3) & 0x7F8u, a1 = (s & 1 ? q >> 21 : q >> 5) & 0x7F8u;
+        uint32_t s8;  // the eight values' signs
+        if constexpr (T == TSX_IQ3_XXS) {
+            const uint32_t s7 = (S.a[s >> 2] >> (7 * (s & 3))) & 127u;
+            s8 = s7 | (uint32_t) __builtin_popcount(s7) << 7;  // bit 7: the parity (and bits above)
+        } else {
+            const uint32_t qh = (uint32_t) R.qh >> (8 * (s >> 2) + 2 * (s & 3));
+            s8 = S.a[s >> 2] >> (8 * (s & 3));
+            a0 |= (qh << 11) & 0x800u;
+            a1 |= (qh << 10) & 0x800u;
+        }
+        const uint32_t m = S.m[s >> 2];
+        const lds_ptr<const uint8_t> stab = (lds_ptr<const uint8_t>) tab + 8 * small_grid<T>();
+        const v2u g0 = *(lds_ptr<const v2u>) (tab + a0) ^ *(lds_ptr<const v2u>) (stab + ((s8 << 3) & 0x78u));
+        const v2u g1 = *(lds_ptr<const v2u>) (tab + a1) ^ *(lds_ptr<const v2u>) (stab + ((s8 >> 1) & 0x78u));
+        f[0] = hmul(g0.x, m);
+        f[1] = hmul(g0.y, m);
+        f[2] = hmul(g1.x, m);
+        f[3] = hmul(g1.y, m);
+    }
+    return v4i{(int) f[0], (int) f[1], (int) f[2], (int) f[3]};
+}
+
+template <int T, bool FUSE>
+__global__ void __launch_bounds__(64 * kSWaves) __attribute__((amdgpu_waves_per_eu(small_wpe<T>())))
+mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t row_bytes, int w_rows, int w_cols,
+                 int n_exp, MmqPlanes P, const int32_t* __restrict__ bounds, const int32_t* __restrict__ ids,
+                 float* __restrict__ dst, int64_t ld_dst, const int32_t* __restrict__ xids, MmqPlanes H, int nbx,
+                 int passes, int vec4) {
+    using L = SmallLds<T>;
+    constexpr int NW = kSWaves, NT = 64 * NW, EPT = kMaxExpertsMmq / NT;
+    constexpr int BH = FUSE ? 16 * NW : 32 * NW;  // output columns per block and pass
+    constexpr bool Q4K = T == TSX_Q4_K;
+    __shared__ __attribute__((aligned(16))) uint8_t s_lds[L::BYTES];
+    auto& s_dw = *reinterpret_cast<float(*)[NW][32]>(s_lds + L::DW);
+    int* const s_ex = reinterpret_cast<int*>(s_lds + L::EX);
+    int* const s_drow = reinterpret_cast<int*>(s_lds + L::DR);
+    float* const s_dm = reinterpret_cast<float*>(s_lds + L::DM);
+    uint64_t* const s_scan = reinterpret_cast<uint64_t*>(s_lds + L::SCAN);
+    int* const s_item = reinterpret_cast<int*>(s_scan + NW);  // expert, first row, rows
+
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int bx = (int) blockIdx.x % nbx;
+
+    // the codebook: this thread's grid entries, stored below
+    constexpr int GE = small_grid<T>(), GPT = GE / NT;
+    uint2 ge[GPT > 0 ? GPT : 1];
+#pragma unroll
+    for (int j = 0; j < GPT; ++j) ge[j] = *(const uint2*) ((T == TSX_IQ3_XXS ? kHalf.xxs : kHalf.s) + 2 * (tid + NT * j));
+
+    // which expert and which of its token tiles, longest tiles first: the full tiles of every expert, then the partial
+    // last tiles of more than 8 rows, of more than 2, and the shorter ones (counts: full in the low 34 bits, the classes
+    // of partial tiles, at most one per expert, in 10 bits each)
+    uint64_t tc[EPT], mine = 0;
+    int b0[EPT], rows[EPT];
+    auto field = [](uint64_t v, int k) { return (int) (k == 0 ? v & 0x3FFFFFFFFull : v >> (24 + 10 * k) & 0x3FFull); };
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+        const int x = EPT * tid + e;
+        b0[e] = bounds[min(x, n_exp)];
+        rows[e] = bounds[min(x + 1, n_exp)] - b0[e];
+        const int rest = rows[e] % kSTok, cl = rest > 8 ? 1 : rest > 2 ? 2 : 3;
+        tc[e] = (uint64_t) (rows[e] / kSTok) | (uint64_t) (rest > 0) << (24 + 10 * cl);
+        mine += tc[e];
+    }
+    uint64_t total;
+    uint64_t start = block_scan<NT>(mine, s_scan, total);
+    int cls = 0, want = (int) (blockIdx.x / (unsigned) nbx);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int n = field(total, k);
+        if (cls == k && want >= n) {
+            want -= n;
+            ++cls;
+        }
+    }
+    if (cls == 4) return;  // the whole block: fewer tiles than the grid's upper bound
+#pragma unroll
+    for (int e = 0; e < EPT; ++e) {
+        const int s0 = field(start, cls), n = field(tc[e], cls);
+        if (s0 <= want && want < s0 + n) {
+            const int t0 = (cls > 0 ? rows[e] / kSTok : want - s0) * kSTok;
+            s_item[0] = EPT * tid + e;
+            s_item[1] = b0[e] + t0;
+            s_item[2] = min(kSTok, rows[e] - t0);
+        }
+        start += tc[e];
+    }
+    if constexpr (GE > 0) {
+#pragma unroll
+        for (int j = 0; j < GPT; ++j) *(lds_ptr<v2u>) (s_lds + L::TAB + 8 * (tid + NT * j)) = v2u{ge[j].x, ge[j].y};
+        // and the masks of four sign bits
+        if (tid < 16)
+            *(lds_ptr<v2u>) (s_lds + L::TAB + 8 * (GE + tid)) =
+                v2u{(tid & 1u) << 15 | (tid >> 1 & 1u) << 31, (tid >> 2 & 1u) << 15 | (uint32_t) (tid >> 3) << 31};
+    }
+    __syncthreads();
+    const int x = __builtin_amdgcn_readfirstlane(s_item[0]), row0 = __builtin_amdgcn_readfirstlane(s_item[1]);
+    const int nr = __builtin_amdgcn_readfirstlane(s_item[2]);
+    const int nu = w_cols / 32, nchunks = w_cols / kChunk;
+    // pass p, tile t, row lr of the wave.  FUSE: gate row col + lr (t = 0) and the up row w_rows further (t = 1), col =
+    // BH (passes bx + p) + 16 wave; else rows col + 16 t + lr, col = BH (passes bx + p) + 32 wave.  A wave past the last
+    // row repeats the last rows and stores nothing
+    constexpr int CW = FUSE ? 16 : 32;
+    constexpr int CB = chunk_bytes<T>();
+    const uint8_t* const we = w + (uint64_t) x * expert_bytes;
+    auto col_of = [&](int p) { return BH * (passes * bx + p) + CW * wave; };
+    auto row_base = [&](int p, int c, int t) -> uint64_t {  // row 0 of the tile, the same in every lane
+        const int col = min(col_of(p), w_rows - CW);
+        return (uint64_t) we + (uint64_t) (uint32_t) (col + (FUSE ? t * w_rows : 16 * t)) * row_bytes + (uint32_t) (c * CB);
+    };
+    const uint32_t lro = lr * row_bytes;
+    const int npass = min(passes, (w_rows - BH * passes * bx + BH - 1) / BH);
+    auto fetch_w = [&](MmqRaw<T> (&R)[2], int p, int c) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const uint64_t b = row_base(p, c, t);
+            raw_load<T>(R[t], gbl_at<uint8_t>(b & ~(uint64_t) 3), lro + (uint32_t) (b & 3), g);
+        }
+    };
+    MmqRaw<T> R[2];  // the next iteration's weights, in flight
+    fetch_w(R, 0, 0);
+
+    // this thread's share of a window: half unit (stok, window chunk sc, unit su, half sh)
+    const int wch = max(1, min(NT / 16 / nr, nchunks)), nwin = (nchunks + wch - 1) / wch;
+    const int ul = tid / nr, stok = tid - ul * nr, sh = ul & 1, su = (ul >> 1) & 7, sc = ul >> 4;
+    int arow = row0 + stok;
+    if (xids) arow = xids[arow];
+    if (!FUSE && tid < nr) s_drow[tid] = ids ? ids[row0 + tid] : row0 + tid;
+    const int8_t* const aq = P.q + (int64_t) arow * P.cols + 32 * su + 16 * sh;
+    const float* const ad = P.d + (int64_t) arow * nu;
+    const int32_t* const am = P.m + (int64_t) arow * nu;
+    auto stage_b = [&](int v) {
+        const int c = v * wch + sc;
+        if (sc >= wch || c >= nchunks) return;
+        const v4i bc = *(const v4i*) (aq + kChunk * c);
+        const float4 x0 = *(const float4*) (ad + 8 * c), x1 = *(const float4*) (ad + 8 * c + 4);
+        const float du = ad[8 * c + su];
+        const float mx = fmaxf(fmaxf(fmaxf(x0.x, x0.y), fmaxf(x0.z, x0.w)), fmaxf(fmaxf(x1.x, x1.y), fmaxf(x1.z, x1.w)));
+        const int e = mx > 0.f ? __builtin_amdgcn_frexp_expf(mx) - 5 : 0;  // mx in [2^(e+4), 2^(e+5))
+        const float dn = __builtin_amdgcn_ldexpf(du, -e);
+        // 1.5 * 2^(10 + the scale's exponent): what a sum with it is rounded to is a multiple of that power of two
+        const float mg = dn > 0.f ? __builtin_amdgcn_ldexpf(1.5f, __builtin_amdgcn_frexp_expf(dn) + 9) : 0.f;
+        const _Float16 dh = (_Float16) dn, mh = (_Float16) mg;
+        const h2 d2 = {dh, dh}, m2 = {mh, mh};
+        uint8_t* const o = s_lds + L::B + (((8 * sc + 4 * (su & 1) + 2 * sh) * 8 + (su >> 1)) * nr + stok) * 16;
+#pragma unroll
+        for (int qq = 0; qq < 2; ++qq) {
+            uint32_t f[4];
+            i8_to_h((uint32_t) bc[2 * qq], f[0], f[1]);
+            i8_to_h((uint32_t) bc[2 * qq + 1], f[2], f[3]);
+            v4i hi, lo;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const h2 cv = __builtin_bit_cast(h2, f[k]);
+                const h2 hv = __builtin_elementwise_fma(cv, d2, m2) - m2;
+                hi[k] = __builtin_bit_cast(int, hv);
+                lo[k] = __builtin_bit_cast(int, __builtin_elementwise_fma(cv, d2, -hv));
+            }
+            *(lds_ptr<v4i>) (o + (8 * qq) * nr * 16) = hi;
+            *(lds_ptr<v4i>) (o + (8 * qq + 4) * nr * 16) = lo;
+        }
+        if (su == 0 && sh == 0) s_ex[sc * nr + stok] = e;
+        if constexpr (Q4K) {
+            if (sh == 0) s_dm[(sc * 8 + su) * nr + stok] = du * (float) am[8 * c + su];
+        }
+    };
+    stage_b(0);
+    __syncthreads();
+
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+    const int tokc = min(lr, nr - 1);  // this lane's token, a row past the last taking the last
+    for (int p = 0; p < npass; ++p) {
+        v4f tot[2] = {zero, zero};
+        int cw = 0;  // the chunk's place in its window
+        for (int c = 0; c < nchunks; ++c, ++cw) {
+            if (nwin > 1 && (cw == wch || (c == 0 && p > 0))) {  // the next window
+                __syncthreads();
+                stage_b(cw == wch ? c / wch : 0);
+                __syncthreads();
+                cw = 0;
+            }
+            // this iteration's weights; the next one's requested (the last one's again after the last)
+            MmqRaw<T> W[2] = {R[0], R[1]};
+            const int sft = Q4K ? 0 : (int) (((uint32_t) row_base(p, c, 0) + lro + 2) & 2) * 8;
+            {
+                const int np = c + 1 < nchunks ? p : min(p + 1, npass - 1);
+                const int nc = c + 1 < nchunks ? c + 1 : p + 1 < npass ? 0 : c;
+                fetch_w(R, np, nc);
+            }
+            MmqScale<T> S[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) raw_scales<T>(W[t], sft, g, S[t]);
+            if (g < 2) s_dw[wave][lane & 31] = g == 0 ? S[0].d : S[1].d;
+            v4f hi[2], lo[2];
+            const uint8_t* const bw = s_lds + L::B + (cw * 8 * 8 + g) * nr * 16 + tokc * 16;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                v4i A[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) A[t] = raw_frag<T>(W[t], S[t], sft, s, s_lds + L::TAB);
+                const v4i bh = *(lds_ptr<const v4i>) (bw + (s * 8) * nr * 16);
+                const v4i bl = *(lds_ptr<const v4i>) (bw + (s * 8 + 4) * nr * 16);
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    hi[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t]), __builtin_bit_cast(v8h, bh),
+                                                                   s == 0 ? zero : hi[t], 0, 0, 0);
+                    lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t]), __builtin_bit_cast(v8h, bl),
+                                                                   s == 0 ? zero : lo[t], 0, 0, 0);
+                }
+            }
+            if constexpr (Q4K) {
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const float bm = s_dm[(cw * 8 + 2 * g + h) * nr + tokc];
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+                        tot[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[t].mn[h], bm, tot[t], 0, 0, 0);
+                }
+            }
+            const float dt = __builtin_amdgcn_ldexpf(1.0f, s_ex[cw * nr + tokc]);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const v4f dw = *(lds_ptr<const v4f>) &s_dw[wave][16 * t + 4 * g];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) tot[t][i] = __builtin_fmaf(hi[t][i] + lo[t][i], dw[i] * dt, tot[t][i]);
+            }
+        }
+        // the pass's outputs
+        const int col = col_of(p);
+        if constexpr (FUSE) {
+#pragma clang fp contract(off)
+            // h = silu(gate) * up (lane: h columns col + 4 g + i, token lr), the product rounded on its own, to LDS (the
+            // activations' place, once every wave is past its last chunk: FUSE takes one pass), then eight lanes a Q8_1
+            // block of it
+            float* const s_h = (float*) (s_lds + L::B);  // [token][BH + 4]
+            constexpr int HS = BH + 4, QR = BH / 4;      // floats and quads of a row
+            const float4 hv = {prompt_swiglu(tot[0][0], tot[1][0]), prompt_swiglu(tot[0][1], tot[1][1]),
+                               prompt_swiglu(tot[0][2], tot[1][2]), prompt_swiglu(tot[0][3], tot[1][3])};
+            __syncthreads();
+            if (lr < nr) *(float4*) (s_h + lr * HS + CW * wave + 4 * g) = hv;
+            __syncthreads();
+            for (int i = tid; i < (nr * QR + 63) / 64 * 64; i += NT) {  // whole waves: reductions inside
+                const int tok = min(i / QR, nr - 1), c4 = i % QR, hc = BH * bx + 4 * c4;
+                const float4 v = *(const float4*) (s_h + tok * HS + 4 * c4);
+                float a = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+                a = lanes_reduce<8>(a, OpMax());
+                const float d = q8_1_scale(a);
+                int qv[4];
+                q8_1_codes4(v, a, d, qv);
+                const float qs = lanes_reduce<8>((float) (qv[0] + qv[1] + qv[2] + qv[3]), OpAddF());  // exact in fp32
+                if (i < nr * QR && hc < w_rows) {
+                    const int64_t hr = row0 + tok;
+                    *(uint32_t*) (H.q + hr * H.cols + hc) = ((uint32_t) qv[0] & 0xFFu) | ((uint32_t) qv[1] & 0xFFu) << 8 |
+                                                            ((uint32_t) qv[2] & 0xFFu) << 16 | ((uint32_t) qv[3] & 0xFFu) << 24;
+                    if ((c4 & 7) == 0) {
+                        H.d[hr * (H.cols / 32) + hc / 32] = h2f(f2h(q8_1_finite(d)));
+                        H.m[hr * (H.cols / 32) + hc / 32] = (int32_t) qs;
+                    }
+                }
+            }
+        } else if (col < w_rows && lr < nr) {
+            // weight row 16 t + 4 g + i of the wave, token lr
+            float* const o = dst + (int64_t) s_drow[lr] * ld_dst + col + 4 * g;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if (vec4) {
+                    *(v4f*) (o + 16 * t) = tot[t];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) o[16 * t + i] = tot[t][i];
+                }
+            }
+        }
+    }
+}
+
+// The few-rows form where a product has at most this many rows per expert on average (the routing's skew is not known
+// here): a layer of 256 experts top-8, IQ3, at 256 tokens 188 -> 157 us with Zipf(1.3) routing, at 400 evenly routed
+// tokens (12.5 rows) 309 -> 217 us, but at 300 skewed ones 155 -> 168; Q4_K, 128 experts, Zipf(1.1): 128 tokens 118 -> 116
+// us, 180 tokens 132 -> 139.  A product over one or a few experts takes it up to kFewRows rows: few blocks in flight, which
+// the 16-row tiles make four times as many of
+constexpr int kFewRowsPerExpert = 8, kFewRows = 64;
+inline bool few_rows(int64_t rows, int64_t experts) {
+    return rows <= std::max<int64_t>(kFewRowsPerExpert * experts, kFewRows);
+}
+inline int64_t small_tiles(int64_t rows, int64_t experts) { return rows / kSTok + std::min(rows, experts); }
+
 __global__ void __launch_bounds__(kThreads) mmq_swiglu_kernel(const float* __restrict__ gu, float* __restrict__ h,
                                                               int64_t rows, int64_t n_ff, int interleaved) {
 #pragma clang fp contract(off)
@@ -1130,6 +1546,21 @@ TSX_API int tsx_moe_mmq_run(const tsx_mmq_product* p, void* stream) {
     if (p->w_cols % kChunk == 0 && p->w_rows % 64 == 0 && p->n <= kMaxExpertsMmq && aligned(p->w, 16) &&
         p->expert_bytes % 16 == 0) {
         const int nw = p->type == TSX_Q4_K && p->w_rows % 128 == 0 ? 4 : p->w_rows % 256 == 0 ? 8 : p->w_rows % 128 == 0 ? 4 : 2;
+        if (p->type != TSX_Q8_0 && few_rows(p->total_rows, p->n)) {
+            if (p->total_rows == 0) return TSX_OK;
+            return with_type(p->type, [&](auto T) {
+                constexpr int TT = decltype(T)::value == TSX_Q8_0 ? TSX_Q4_K : decltype(T)::value;
+                // two passes of a short row (a down product) share a block's set-up and activations
+                const int passes = p->w_cols <= 1024 ? 2 : 1, per = 32 * kSWaves * passes;
+                const int nbx = (int) ((p->w_rows + per - 1) / per);
+                mmq_small_kernel<TT, false>
+                    <<<(unsigned) (nbx * small_tiles(p->total_rows, p->n)), 64 * kSWaves, 0, s>>>(
+                        (const uint8_t*) p->w, p->expert_bytes, (uint32_t) rb, (int) p->w_rows, (int) p->w_cols, p->n, P,
+                        p->bounds, p->ids, p->dst, p->ld_dst, nullptr, MmqPlanes{}, nbx, passes,
+                        aligned(p->dst, 16) && p->ld_dst % 4 == 0);
+                return launch_status("tsx_moe_mmq_run/mfma");
+            });
+        }
         return with_type(p->type, [&](auto T) {
             constexpr int TT = decltype(T)::value;
             const int64_t max_tiles = xcd_tiles((p->total_rows + bn_of<TT>() - 1) / bn_of<TT>() + p->n);
@@ -1182,6 +1613,15 @@ TSX_API int tsx_moe_mmq_gate_up_swiglu(const void* w, int type, int64_t n_ff, in
     if (n_exp == 0 || n_rows == 0) return TSX_OK;
     const MmqPlanes P = planes((void*) xq, x_rows, n_embd), H = planes(hq, n_rows, n_ff);
     const hipStream_t s = (hipStream_t) stream;
+    if (type != TSX_Q8_0 && few_rows(n_rows, n_exp))
+        return with_type(type, [&](auto T) {
+            constexpr int TT = decltype(T)::value == TSX_Q8_0 ? TSX_Q4_K : decltype(T)::value;
+            const int nbx = (int) ((n_ff + 16 * kSWaves - 1) / (16 * kSWaves));
+            mmq_small_kernel<TT, true><<<(unsigned) (nbx * small_tiles(n_rows, n_exp)), 64 * kSWaves, 0, s>>>(
+                (const uint8_t*) w, expert_bytes, (uint32_t) rb, (int) n_ff, (int) n_embd, n_exp, P, bounds, nullptr,
+                nullptr, 0, xids, H, nbx, 1, 0);
+            return launch_status("tsx_moe_mmq_gate_up_swiglu");
+        });
     return with_type(type, [&](auto T) {
         constexpr int BN = bn_of<decltype(T)::value>();
         const int64_t max_tiles = xcd_tiles((n_rows + BN - 1) / BN + n_exp);
