@@ -181,6 +181,20 @@ def test_decode_layer_edges(case):
     assert err < 1e-3
 
 
+@pytest.mark.parametrize("T", [1, 3, 6])
+@pytest.mark.parametrize("FF", [128, 384])
+def test_decode_layer_q8_0_odd_row_pieces(FF, T):
+    """Q8_0 down rows of an odd number of 8-byte pieces (136 and 408 bytes): rows and units start at every even offset of
+    a 16-byte piece in the LDS slabs."""
+    gu, d, N, E, k, shared = Q8_0, Q8_0, 512, 64, 4, True
+    L, p, order, W = make_layer(gu, d, N, FF, E, shared, distinct=5, seed=4)
+    x, logits, sgate = inputs("edge", T, E, N, seed=FF + T)
+    got, ids = run_layer(W, k, x, logits, sgate)
+    y0, eids, _ = O.moe_layer(0, O.layout(gu, d, N, FF), x, logits, k, p[order], p.shape[1], p[len(p) - 1], sgate)
+    assert (ids == eids).all()
+    assert rel_l2(got, y0) < 1e-3
+
+
 def test_decode_layer_residual_alias_and_replay():
     """y may alias x (x <- x + moe(x)); a captured graph replays to the same bits as the eager call, every time."""
     gu, d, N, FF, E, k, shared, T = CONFIGS["c3_verify_iq3"]
