@@ -314,7 +314,7 @@ template <int T, int NW, int NB> struct F16Layout {
     static constexpr int DL = RHO + lds_round(NB * 8 * 16 * RS * 4);
     static constexpr int DM = DL + lds_round(BN * 4);
     static constexpr int SCAN = DM + lds_round((Q4K ? NB * 8 * (BN + 16) : 1) * 4);
-    static constexpr int DR = SCAN + lds_round((NW + 1) * 8);
+    static constexpr int DR = SCAN + lds_round((NW + 2) * 8);
     static constexpr int RAW = DR + lds_round(BN * 4);
     static constexpr int TB = RAW + lds_round(NW * 32 * raw_stride<T>());
     static constexpr int BYTES = TB + NB * BN * kBStride * 2;
@@ -414,8 +414,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     // 32-lane half read different banks
     auto& s_dm = *reinterpret_cast<float(*)[Q4K ? NB : 1][8][Q4K ? kBN + 16 : 1]>(s_lds + L::DM);
     uint64_t* const s_scan = reinterpret_cast<uint64_t*>(s_lds + L::SCAN);
-    int& s_x = reinterpret_cast<int*>(s_scan + NW)[0];
-    int& s_tile0 = reinterpret_cast<int*>(s_scan + NW)[1];
+    int* const s_item = reinterpret_cast<int*>(s_scan + NW);  // expert, first row, rows
     int* const s_drow = reinterpret_cast<int*>(s_lds + L::DR);  // the output row of each token of the tile
     auto& s_raw = *reinterpret_cast<uint8_t(*)[NW][32 * RS]>(s_lds + L::RAW);
     auto& tB = *reinterpret_cast<_Float16(*)[NB][kBN * kBStride]>(s_lds + L::TB);
@@ -439,13 +438,15 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     // more than kBN / 2 rows, of more than kBN / 4, and the shorter ones.  Counts travel packed in four 16-bit fields
     // (a total is at most gridDim.y < 2^16)
     uint64_t tc[EPT], mine = 0;
+    int b0[EPT], rows[EPT];
 #pragma unroll
     for (int e = 0; e < EPT; ++e) {
         const int x = EPT * tid + e;
-        const int b0 = bounds[min(x, n_exp)], b1 = bounds[min(x + 1, n_exp)];
-        const int rows = x < n_exp ? b1 - b0 : 0, rest = rows % kBN;
+        b0[e] = bounds[min(x, n_exp)];
+        rows[e] = bounds[min(x + 1, n_exp)] - b0[e];
+        const int rest = rows[e] % kBN;
         const int cl = rest > kBN / 2 ? 1 : rest > kBN / 4 ? 2 : 3;  // the partial tile's field
-        tc[e] = (uint64_t) (rows / kBN) | (uint64_t) (rest > 0) << (16 * cl);
+        tc[e] = (uint64_t) (rows[e] / kBN) | (uint64_t) (rest > 0) << (16 * cl);
         mine += tc[e];
     }
     uint64_t total;
@@ -477,15 +478,18 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
     for (int e = 0; e < EPT; ++e) {
         const int s0 = (int) (start >> (16 * cls) & 0xFFFF), n = (int) (tc[e] >> (16 * cls) & 0xFFFF);
         if (s0 <= want && want < s0 + n) {
-            s_x = EPT * tid + e;
-            s_tile0 = cls > 0 ? (int) (tc[e] & 0xFFFF) : want - s0;  // the tile's index within its expert
+            const int t0 = (cls > 0 ? rows[e] / kBN : want - s0) * kBN;  // the tile's first row within its expert
+            s_item[0] = EPT * tid + e;
+            s_item[1] = b0[e] + t0;
+            s_item[2] = min(kBN, rows[e] - t0);
         }
         start += tc[e];
     }
     __syncthreads();
-    const int x = s_x;
-    const int row0 = bounds[x] + s_tile0 * kBN;
-    const int nrows = min(kBN, bounds[x + 1] - row0);
+    // (handed over whole, rather than the expert alone and its bounds read again: a round trip less in every block, 0.5 %
+    // of a launch)
+    const int x = __builtin_amdgcn_readfirstlane(s_item[0]), row0 = __builtin_amdgcn_readfirstlane(s_item[1]);
+    const int nrows = __builtin_amdgcn_readfirstlane(s_item[2]);
     const int ntt = (nrows + 15) >> 4;  // 16-token MFMA tiles with rows in them
     const int wrow = FUSE ? (BM / 2) * bx + 16 * wave : bx * CP * BM + 32 * wave;
     const uint8_t* wbase = w + (uint64_t) x * expert_bytes + (uint64_t) wrow * row_bytes;
