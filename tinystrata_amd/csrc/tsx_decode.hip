@@ -79,7 +79,7 @@ __device__ __forceinline__ void row_dots(const uint8_t* const (&rows)[R], const 
 #pragma unroll
     for (int j = 0; j < R; ++j)
 #pragma unroll
-        for (int c = 0; c < NC; ++c) acc[j][c] = lanes_sum<LPR>(acc[j][c]);  // (every lane of the wave calls)
+        for (int c = 0; c < NC; ++c) acc[j][c] = tree_sum<LPR>(acc[j][c]);  // (every lane of the wave calls)
 }
 // Rows per wave and pass: R of each LPR-lane group, as many of 4, 2 and 1 as leave kRowsPerWaveMin waves, eight a CU.
 // Several rows share a unit's activation loads and a block's chain of table reads; with fewer waves than that more waves

@@ -534,6 +534,29 @@ __device__ __forceinline__ float lanes_sum(float v) {
     return lanes_reduce<W>(v, OpAddF());
 }
 
+// group_sum's tree (lanes W / 2, .., 2, 1 apart) bit for bit, without LDS permutes: the lane-swap and row-rotate forms of
+// its steps (after the sum of lanes 8 apart a rotate by 4 is the exchange of lanes 4 apart).  All 64 lanes must be active
+template <int W>
+__device__ __forceinline__ float tree_sum(float v) {
+    static_assert(W >= 1 && W <= 64 && (W & (W - 1)) == 0, "tree_sum width");
+    if constexpr (W >= 64) {
+        const uint32_t b = __builtin_bit_cast(uint32_t, v);
+        const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+        v = __builtin_bit_cast(float, (uint32_t) r[0]) + __builtin_bit_cast(float, (uint32_t) r[1]);
+    }
+    if constexpr (W >= 32) {
+        const uint32_t b = __builtin_bit_cast(uint32_t, v);
+        const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+        v = __builtin_bit_cast(float, (uint32_t) r[0]) + __builtin_bit_cast(float, (uint32_t) r[1]);
+    }
+    if constexpr (W >= 16) v += dpp_mov<0x128>(v);
+    if constexpr (W >= 16) v += dpp_mov<0x124>(v);
+    else if constexpr (W == 8) v += __shfl_xor(v, 4, 8);
+    if constexpr (W >= 4) v += dpp_mov<0x4E>(v);
+    if constexpr (W >= 2) v += dpp_mov<0xB1>(v);
+    return v;
+}
+
 // ------------------------------------------------------------------ wave argmax on (value, id) keys
 // A float's order as an unsigned word (larger float -> larger word; -inf below -FLT_MAX below every probability).
 __device__ __forceinline__ uint32_t ord_key(float f) {
