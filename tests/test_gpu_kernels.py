@@ -430,7 +430,7 @@ def test_mmq_run_tile_classes(t):
 FEW_COUNTS = [0, 1, 2, 3, 5, 16, 17, 33, 0, 8, 4, 1]  # at most eight rows per expert on average
 
 
-@pytest.mark.parametrize("t", [IQ3_XXS, IQ3_S, Q4_K])
+@pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("w_cols,w_rows,pad", [(256, 64, 0), (512, 448, 1), (768, 320, 0), (2048, 128, 0), (1280, 192, 3)])
 def test_mmq_run_few_rows(t, w_cols, w_rows, pad):
     """The few-rows form: experts of 0 to 33 rows (tiles of 1 to 16 rows, whose windows hold 16 chunks down to one), odd
@@ -469,7 +469,7 @@ def test_mmq_run_few_rows(t, w_cols, w_rows, pad):
     assert (np.abs(got[:, :w_rows] - exp) <= 1e-5 * np.abs(exp) + 1e-5 * scale).all()
 
 
-@pytest.mark.parametrize("t", [IQ3_XXS, IQ3_S, Q4_K])
+@pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("N,FF,counts", [(512, 128, FEW_COUNTS), (2048, 384, FEW_COUNTS), (768, 256, [64]), (256, 128, [1])])
 def test_mmq_gate_up_swiglu_few_rows(t, N, FF, counts):
     """The few-rows form of the fused gate/up launch against the call sequence on the GPU: the same planes byte for

@@ -1051,21 +1051,36 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
 // that share a CU.
 constexpr int kSTok = 16;
 constexpr int kSWaves = 4;  // per block
-constexpr int kSWindow = 64 * 64 * kSWaves;  // LDS bytes of a window: a half unit of 16 codes per thread
-// waves per SIMD that the registers are held to: four for the codebook formats (128 registers, no spills), three for
-// Q4_K, whose raw rows are wider (at four it spills: a batch of 32, gate/up and down 126 -> 117 us a layer with three)
-template <int T> constexpr int small_wpe() { return T == TSX_Q4_K ? 3 : 4; }
+constexpr int kSWindow = 64 * 64 * kSWaves;  // LDS bytes of a window: a half unit of 16 codes per thread (Q8_0: four)
+constexpr int kSUnitRow = 40;                // Q8_0: floats from unit to unit of the rows' scales (distinct banks)
+//
+// Q8_0 has a float scale per unit, which stays outside: a unit's dot product is an integer of its own (the int8 MFMA
+// 16x16x64), times the two scales' exact product.  The lane groups keep units of their own all the same, and with them 68
+// consecutive bytes a row: the MFMA's columns are four tokens times the four lane groups' units, column 4 i + k holding
+// token k's codes in lane group i and zeros in the others, so that two steps of 16 values finish four units at once.
+// Every four tokens of the tile are a set of columns; at the end a token's four unit columns are added.
+// 60 tokens (128 experts top-8, 768 x 2048): two layers 444 -> 341 us (3.7 TB/s of weights); 16 tokens 169 -> 131 us a
+// layer.  At two waves per SIMD it takes 220 registers; held to three or four it spills 68 and 204 of them.
+//
+// waves per SIMD that the registers are held to: two for Q8_0, four for the codebook formats (128 registers, no spills),
+// three for Q4_K, whose raw rows are wider (at four it spills: a batch of 32, gate/up and down 126 -> 117 us a layer with
+// three)
+template <int T> constexpr int small_wpe() { return T == TSX_Q8_0 ? 2 : T == TSX_Q4_K ? 3 : 4; }
 template <int T> constexpr int small_grid() { return T == TSX_IQ3_XXS ? 256 : T == TSX_IQ3_S ? 512 : 0; }
 // the codebook (four fp16 magnitudes an entry) and the sixteen masks of four sign bits
 template <int T> constexpr int small_tab_bytes() { return small_grid<T>() > 0 ? 8 * small_grid<T>() + 128 : 0; }
 template <int T> struct SmallLds {
     static constexpr int TAB = 0, B = TAB + small_tab_bytes<T>();
-    static constexpr int DW = B + kSWindow;                // float [kSWaves][32]: the rows' scales of the chunk
-    static constexpr int EX = DW + kSWaves * 128;          // int [chunk of the window][token]: the exponents
+    static constexpr bool Q80 = T == TSX_Q8_0;
+    static constexpr int DW = B + kSWindow + (Q80 ? 16 * kSTok : 0);  // (Q8_0: a token's codes end in 16 bytes of padding)
+    // the rows' scales of the chunk: float [kSWaves][32]; Q8_0: [kSWaves][unit][kSUnitRow]
+    static constexpr int EX = DW + kSWaves * (Q80 ? 8 * kSUnitRow * 4 : 128);
+    // int [chunk of the window][token]: the exponents; Q8_0: 64 bytes of zeros
     static constexpr int DR = EX + kSWindow / 1024 * 4;    // int [kSTok]: the token's output row
     static constexpr int SCAN = DR + kSTok * 4;
     static constexpr int DM = SCAN + (kSWaves + 2) * 8;    // Q4_K: float [chunk][unit][token]: min-term factors
-    static constexpr int BYTES = DM + (T == TSX_Q4_K ? kSWindow / 1024 * 8 * 4 : 0);
+    // (Q8_0: float [token][unit of the window]: the activations' scales)
+    static constexpr int BYTES = DM + (Q80 ? kSWindow / 256 * 8 * 4 : T == TSX_Q4_K ? kSWindow / 1024 * 8 * 4 : 0);
 };
 
 typedef uint32_t v2u __attribute__((ext_vector_type(2)));
@@ -1076,6 +1091,7 @@ template <int T> struct MmqRaw;
 template <> struct MmqRaw<TSX_IQ3_XXS> { v4i q; int q4; v2i a; int a2; uint16_t d; };
 template <> struct MmqRaw<TSX_IQ3_S> { v4i q; int q4; v2i a; int a2; uint16_t qh, d; uint8_t sc; };
 template <> struct MmqRaw<TSX_Q4_K> { v4i h, q[2]; };
+template <> struct MmqRaw<TSX_Q8_0> { v4i q[4]; int q4; };  // two units whole: {scale, 32 codes} twice
 // the row's block of the chunk lies at base + o (base 4-byte aligned and the same in every lane); lane group g takes
 // units 2 g and 2 g + 1
 template <int T> __device__ __forceinline__ void raw_load(MmqRaw<T>& R, gbl_ptr<const uint8_t> base, uint32_t o, int g) {
@@ -1083,6 +1099,10 @@ template <int T> __device__ __forceinline__ void raw_load(MmqRaw<T>& R, gbl_ptr<
         R.h = *(gbl_ptr<const v4i>) (base + o);
         R.q[0] = *(gbl_ptr<const v4i>) (base + (o + 16 + 32 * g));
         R.q[1] = *(gbl_ptr<const v4i>) (base + (o + 32 + 32 * g));
+    } else if constexpr (T == TSX_Q8_0) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) R.q[k] = *(gbl_ptr<const v4i_a4>) (base + (o + 68 * g + 16 * k));
+        R.q4 = *(gbl_ptr<const int>) (base + (o + 68 * g + 64));
     } else {
         // the words that hold the lane's bytes: they start on a 2-byte boundary, and where that is a 4-byte one the
         // extra word is the last one again
@@ -1179,9 +1199,11 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
     using L = SmallLds<T>;
     constexpr int NW = kSWaves, NT = 64 * NW, EPT = kMaxExpertsMmq / NT;
     constexpr int BH = FUSE ? 16 * NW : 32 * NW;  // output columns per block and pass
-    constexpr bool Q4K = T == TSX_Q4_K;
+    constexpr bool Q4K = T == TSX_Q4_K, Q80 = T == TSX_Q8_0;
+    constexpr int PPT = Q80 ? 4 : 1;  // 16-code pieces of a window per thread
     __shared__ __attribute__((aligned(16))) uint8_t s_lds[L::BYTES];
     auto& s_dw = *reinterpret_cast<float(*)[NW][32]>(s_lds + L::DW);
+    auto& s_uw = *reinterpret_cast<float(*)[NW][8][kSUnitRow]>(s_lds + L::DW);  // Q8_0
     int* const s_ex = reinterpret_cast<int*>(s_lds + L::EX);
     int* const s_drow = reinterpret_cast<int*>(s_lds + L::DR);
     float* const s_dm = reinterpret_cast<float*>(s_lds + L::DM);
@@ -1272,7 +1294,7 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
     fetch_w(R, 0, 0);
 
     // this thread's share of a window: half unit (stok, window chunk sc, unit su, half sh)
-    const int wch = max(1, min(NT / 16 / nr, nchunks)), nwin = (nchunks + wch - 1) / wch;
+    const int wch = max(1, min(PPT * NT / 16 / nr, nchunks)), nwin = (nchunks + wch - 1) / wch;
     const int ul = tid / nr, stok = tid - ul * nr, sh = ul & 1, su = (ul >> 1) & 7, sc = ul >> 4;
     int arow = row0 + stok;
     if (xids) arow = xids[arow];
@@ -1280,7 +1302,36 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
     const int8_t* const aq = P.q + (int64_t) arow * P.cols + 32 * su + 16 * sh;
     const float* const ad = P.d + (int64_t) arow * nu;
     const int32_t* const am = P.m + (int64_t) arow * nu;
-    auto stage_b = [&](int v) {
+    // Q8_0: the window's codes as they are, [token][chunk][unit] 32 bytes and 16 of padding per token, and the scales
+    // behind them; a thread's pieces and its four scales stay those of the same tokens in every window
+    const int tstride = 256 * wch + 16;
+    int ptok[PPT], prow[PPT], stok8 = 0, srow8 = 0;
+    if constexpr (Q80) {
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) {
+            ptok[k] = min((tid + NT * k) / (16 * wch), nr - 1);
+            prow[k] = xids ? xids[row0 + ptok[k]] : row0 + ptok[k];
+        }
+        stok8 = min(tid / (2 * wch), nr - 1);
+        srow8 = xids ? xids[row0 + stok8] : row0 + stok8;
+        if (tid < 4) *(lds_ptr<v4i>) (s_lds + L::EX + 16 * tid) = v4i{0, 0, 0, 0};
+    }
+    auto stage_q80 = [&](int v) {
+        v4i q[PPT];
+#pragma unroll
+        for (int k = 0; k < PPT; ++k) {  // chunks past the last take the last one's
+            const int pc = tid + NT * k - 16 * wch * ptok[k], c = min(v * wch + (pc >> 4), nchunks - 1);
+            q[k] = *(const v4i*) (P.q + (int64_t) prow[k] * P.cols + kChunk * c + 16 * (pc & 15));
+        }
+        const int sp = tid - 2 * wch * stok8, cs = min(v * wch + (sp >> 1), nchunks - 1);
+        const float4 d = *(const float4*) (P.d + (int64_t) srow8 * nu + 8 * cs + 4 * (sp & 1));
+#pragma unroll
+        for (int k = 0; k < PPT; ++k)
+            if (tid + NT * k < 16 * wch * nr)
+                *(lds_ptr<v4i>) (s_lds + L::B + ptok[k] * tstride + 16 * (tid + NT * k - 16 * wch * ptok[k])) = q[k];
+        if (tid < 2 * wch * nr) *(float4*) (s_dm + 8 * wch * stok8 + 4 * sp) = d;
+    };
+    auto stage_f16 = [&](int v) {
         const int c = v * wch + sc;
         if (sc >= wch || c >= nchunks) return;
         const v4i bc = *(const v4i*) (aq + kChunk * c);
@@ -1315,6 +1366,10 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
             if (sh == 0) s_dm[(sc * 8 + su) * nr + stok] = du * (float) am[8 * c + su];
         }
     };
+    auto stage_b = [&](int v) {
+        if constexpr (Q80) stage_q80(v);
+        else stage_f16(v);
+    };
     stage_b(0);
     __syncthreads();
 
@@ -1322,6 +1377,11 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
     const int tokc = min(lr, nr - 1);  // this lane's token, a row past the last taking the last
     for (int p = 0; p < npass; ++p) {
         v4f tot[2] = {zero, zero};
+        v4f part[Q80 ? kSTok / 4 : 1][2];  // Q8_0: per set of four tokens, row 4 g + i by column
+        if constexpr (Q80) {
+#pragma unroll
+            for (int s = 0; s < kSTok / 4; ++s) part[s][0] = part[s][1] = zero;
+        }
         int cw = 0;  // the chunk's place in its window
         for (int c = 0; c < nchunks; ++c, ++cw) {
             if (nwin > 1 && (cw == wch || (c == 0 && p > 0))) {  // the next window
@@ -1338,43 +1398,99 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
                 const int nc = c + 1 < nchunks ? c + 1 : p + 1 < npass ? 0 : c;
                 fetch_w(R, np, nc);
             }
-            MmqScale<T> S[2];
-#pragma unroll
-            for (int t = 0; t < 2; ++t) raw_scales<T>(W[t], sft, g, S[t]);
-            if (g < 2) s_dw[wave][lane & 31] = g == 0 ? S[0].d : S[1].d;
-            v4f hi[2], lo[2];
-            const uint8_t* const bw = s_lds + L::B + (cw * 8 * 8 + g) * nr * 16 + tokc * 16;
-#pragma unroll
-            for (int s = 0; s < 8; ++s) {
-                v4i A[2];
-#pragma unroll
-                for (int t = 0; t < 2; ++t) A[t] = raw_frag<T>(W[t], S[t], sft, s, s_lds + L::TAB);
-                const v4i bh = *(lds_ptr<const v4i>) (bw + (s * 8) * nr * 16);
-                const v4i bl = *(lds_ptr<const v4i>) (bw + (s * 8 + 4) * nr * 16);
+            if constexpr (Q80) {
+                const int ci = lr >> 2;  // the lane group whose units this lane's column holds
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    hi[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t]), __builtin_bit_cast(v8h, bh),
-                                                                   s == 0 ? zero : hi[t], 0, 0, 0);
-                    lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t]), __builtin_bit_cast(v8h, bl),
-                                                                   s == 0 ? zero : lo[t], 0, 0, 0);
+                    s_uw[wave][2 * g][16 * t + lr] = h2f((uint16_t) W[t].q[0][0]);
+                    s_uw[wave][2 * g + 1][16 * t + lr] = h2f((uint16_t) ((uint32_t) W[t].q[2][0] >> 16));
+                }
+                wave_lds_order();
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    auto word = [&](int k) { return k == 16 ? W[t].q4 : W[t].q[(k >> 2) & 3][k & 3]; };
+                    v4i A[2][2];  // [unit][half]
+                    v4f dw[2];
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        A[0][k >> 2][k & 3] = (int) __builtin_amdgcn_alignbit((uint32_t) word(k + 1), (uint32_t) word(k), 16);
+                        A[1][k >> 2][k & 3] = word(9 + k);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) dw[j] = *(lds_ptr<const v4f>) &s_uw[wave][2 * ci + j][16 * t + 4 * g];
+#pragma unroll
+                    for (int s = 0; s < kSTok / 4; ++s) {
+                        if (4 * s >= nr) break;  // the same in every lane
+                        const int tok = min(4 * s + (lr & 3), nr - 1);
+                        const uint8_t* const b = s_lds + (ci == g ? L::B + tok * tstride + 256 * cw + 64 * g : L::EX);
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) {
+                            const v4i b0 = *(lds_ptr<const v4i>) (b + 32 * j), b1 = *(lds_ptr<const v4i>) (b + 32 * j + 16);
+                            const float dx = s_dm[8 * wch * tok + 8 * cw + 2 * ci + j];
+                            v4i C = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[j][0], b0, v4i{0, 0, 0, 0}, 0, 0, 0);
+                            C = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[j][1], b1, C, 0, 0, 0);
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                part[s][t][i] = __builtin_fmaf((float) C[i], dw[j][i] * dx, part[s][t][i]);
+                        }
+                    }
+                }
+                wave_lds_order();  // the next chunk's scales go to the same place
+            } else {
+                MmqScale<T> S[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) raw_scales<T>(W[t], sft, g, S[t]);
+                if (g < 2) s_dw[wave][lane & 31] = g == 0 ? S[0].d : S[1].d;
+                v4f hi[2], lo[2];
+                const uint8_t* const bw = s_lds + L::B + (cw * 8 * 8 + g) * nr * 16 + tokc * 16;
+#pragma unroll
+                for (int s = 0; s < 8; ++s) {
+                    v4i A[2];
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) A[t] = raw_frag<T>(W[t], S[t], sft, s, s_lds + L::TAB);
+                    const v4i bh = *(lds_ptr<const v4i>) (bw + (s * 8) * nr * 16);
+                    const v4i bl = *(lds_ptr<const v4i>) (bw + (s * 8 + 4) * nr * 16);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        hi[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t]), __builtin_bit_cast(v8h, bh),
+                                                                       s == 0 ? zero : hi[t], 0, 0, 0);
+                        lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t]), __builtin_bit_cast(v8h, bl),
+                                                                       s == 0 ? zero : lo[t], 0, 0, 0);
+                    }
+                }
+                if constexpr (Q4K) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const float bm = s_dm[(cw * 8 + 2 * g + h) * nr + tokc];
+#pragma unroll
+                        for (int t = 0; t < 2; ++t)
+                            tot[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[t].mn[h], bm, tot[t], 0, 0, 0);
+                    }
+                }
+                const float dt = __builtin_amdgcn_ldexpf(1.0f, s_ex[cw * nr + tokc]);
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const v4f dw = *(lds_ptr<const v4f>) &s_dw[wave][16 * t + 4 * g];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) tot[t][i] = __builtin_fmaf(hi[t][i] + lo[t][i], dw[i] * dt, tot[t][i]);
                 }
             }
-            if constexpr (Q4K) {
+        }
+        if constexpr (Q80) {
+            // the token's four columns, 4 apart, then set lr / 4's sums: token lr, the same lane for every row
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const float bm = s_dm[(cw * 8 + 2 * g + h) * nr + tokc];
+            for (int s = 0; s < kSTok / 4; ++s)
+                if (4 * s < nr) {
 #pragma unroll
                     for (int t = 0; t < 2; ++t)
-                        tot[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[t].mn[h], bm, tot[t], 0, 0, 0);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            float v = part[s][t][i];
+                            v += dpp_mov<0x128>(v);  // row_ror 8
+                            v += dpp_mov<0x124>(v);  // row_ror 4
+                            if (s == lr >> 2) tot[t][i] = v;
+                        }
                 }
-            }
-            const float dt = __builtin_amdgcn_ldexpf(1.0f, s_ex[cw * nr + tokc]);
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const v4f dw = *(lds_ptr<const v4f>) &s_dw[wave][16 * t + 4 * g];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) tot[t][i] = __builtin_fmaf(hi[t][i] + lo[t][i], dw[i] * dt, tot[t][i]);
-            }
         }
         // the pass's outputs
         const int col = col_of(p);
@@ -1428,7 +1544,8 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
 // The few-rows form where a product has at most this many rows per expert on average (the routing's skew is not known
 // here): a layer of 256 experts top-8, IQ3, at 256 tokens 188 -> 157 us with Zipf(1.3) routing, at 400 evenly routed
 // tokens (12.5 rows) 309 -> 217 us, but at 300 skewed ones 155 -> 168; Q4_K, 128 experts, Zipf(1.1): 128 tokens 118 -> 116
-// us, 180 tokens 132 -> 139.  A product over one or a few experts takes it up to kFewRows rows: few blocks in flight, which
+// us, 180 tokens 132 -> 139.  Q8_0, 128 experts, evenly routed: 128 tokens 237 -> 199 us, 256 tokens (16 rows) 254 -> 253,
+// 512 tokens 283 -> 364; Zipf(1.3), 256 experts: 256 tokens 158 -> 150 us, 512 tokens (16 rows) 194 -> 225.  A product over one or a few experts takes it up to kFewRows rows: few blocks in flight, which
 // the 16-row tiles make four times as many of
 constexpr int kFewRowsPerExpert = 8, kFewRows = 64;
 inline bool few_rows(int64_t rows, int64_t experts) {
@@ -1550,10 +1667,10 @@ TSX_API int tsx_moe_mmq_run(const tsx_mmq_product* p, void* stream) {
     if (p->w_cols % kChunk == 0 && p->w_rows % 64 == 0 && p->n <= kMaxExpertsMmq && aligned(p->w, 16) &&
         p->expert_bytes % 16 == 0) {
         const int nw = p->type == TSX_Q4_K && p->w_rows % 128 == 0 ? 4 : p->w_rows % 256 == 0 ? 8 : p->w_rows % 128 == 0 ? 4 : 2;
-        if (p->type != TSX_Q8_0 && few_rows(p->total_rows, p->n)) {
+        if (few_rows(p->total_rows, p->n)) {
             if (p->total_rows == 0) return TSX_OK;
             return with_type(p->type, [&](auto T) {
-                constexpr int TT = decltype(T)::value == TSX_Q8_0 ? TSX_Q4_K : decltype(T)::value;
+                constexpr int TT = decltype(T)::value;
                 // two passes of a short row (a down product) share a block's set-up and activations
                 const int passes = p->w_cols <= 1024 ? 2 : 1, per = 32 * kSWaves * passes;
                 const int nbx = (int) ((p->w_rows + per - 1) / per);
@@ -1617,9 +1734,9 @@ TSX_API int tsx_moe_mmq_gate_up_swiglu(const void* w, int type, int64_t n_ff, in
     if (n_exp == 0 || n_rows == 0) return TSX_OK;
     const MmqPlanes P = planes((void*) xq, x_rows, n_embd), H = planes(hq, n_rows, n_ff);
     const hipStream_t s = (hipStream_t) stream;
-    if (type != TSX_Q8_0 && few_rows(n_rows, n_exp))
+    if (few_rows(n_rows, n_exp))
         return with_type(type, [&](auto T) {
-            constexpr int TT = decltype(T)::value == TSX_Q8_0 ? TSX_Q4_K : decltype(T)::value;
+            constexpr int TT = decltype(T)::value;
             const int nbx = (int) ((n_ff + 16 * kSWaves - 1) / (16 * kSWaves));
             mmq_small_kernel<TT, true><<<(unsigned) (nbx * small_tiles(n_rows, n_exp)), 64 * kSWaves, 0, s>>>(
                 (const uint8_t*) w, expert_bytes, (uint32_t) rb, (int) n_ff, (int) n_embd, n_exp, P, bounds, nullptr,
