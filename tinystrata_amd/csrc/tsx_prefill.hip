@@ -1060,7 +1060,8 @@ constexpr int kSUnitRow = 40;                // Q8_0: floats from unit to unit o
 // token k's codes in lane group i and zeros in the others, so that two steps of 16 values finish four units at once.
 // Every four tokens of the tile are a set of columns; at the end a token's four unit columns are added.
 // 60 tokens (128 experts top-8, 768 x 2048): two layers 444 -> 341 us (3.7 TB/s of weights); 16 tokens 169 -> 131 us a
-// layer.  At two waves per SIMD it takes 220 registers; held to three or four it spills 68 and 204 of them.
+// layer; relative error against 64 bits over 768 columns 2.8e-7 -> 6.2e-8, over 2048 4.9e-7 -> 8.2e-8.  At two waves
+// per SIMD it takes 220 registers; held to three or four waves it spills 68 and 204 of them.
 //
 // waves per SIMD that the registers are held to: two for Q8_0, four for the codebook formats (128 registers, no spills),
 // three for Q4_K, whose raw rows are wider (at four it spills: a batch of 32, gate/up and down 126 -> 117 us a layer with
