@@ -67,6 +67,56 @@ def test_mmvq_matrix_on_a_4_byte_boundary(t, shift):
 
 
 @pytest.mark.parametrize("t", ALL)
+@pytest.mark.parametrize("shift", [1, 2, 3, 7])
+def test_products_on_any_byte_address(t, shift):
+    """Weights that start off a 4-byte boundary - a matrix, an id-indexed offset, a group's blob, experts an odd number of
+    bytes apart - give the bits of the same weights on a 256-byte boundary."""
+    n_in, n_out = 768, 21
+    print(f"byte address t={t} shift={shift}", flush=True)
+    w = weights(t, n_out, n_in, 400 + t)
+    xq = O.quantize_q8_1(np.random.default_rng(t).normal(0, 1, (3, n_in)).astype(np.float32))
+    buf = torch.zeros(w.size + shift + 16, dtype=torch.uint8, device="cuda")
+    buf[shift:shift + w.size] = dev(w.ravel())
+    exp = host(ops.iq_mmvq(t, dev(w), dev(xq), n_in, n_out, 3))
+    assert np.array_equal(host(ops.iq_mmvq(t, buf[shift:], dev(xq), n_in, n_out, 3)), exp)
+    table = torch.tensor([buf.data_ptr()], dtype=torch.int64, device="cuda")
+    y = torch.full((3, n_out), 7.0, device="cuda")
+    ops.mmvq_ids(t, table, torch.zeros(3, dtype=torch.int32, device="cuda"), shift, dev(xq), n_in // 32 * 36, 1, y, n_out, 3,
+                 n_in, n_out)
+    assert np.array_equal(host(y), exp)
+    if t in (Q4_0, Q6_K):
+        return
+    # two experts of the prompt's row-dot product, w.size + shift bytes apart
+    blob = torch.zeros(2 * w.size + 2 * shift + 16, dtype=torch.uint8, device="cuda")
+    blob[:w.size] = dev(w.ravel())
+    blob[w.size + shift:2 * w.size + shift] = dev(w[::-1].copy().ravel())
+    x = torch.randn((4, n_in), generator=torch.Generator(device="cuda").manual_seed(t), device="cuda")
+    xm = ops.mmq_quantize(x, None, t, n_in, n_in, 4)
+    bounds = torch.tensor([0, 2, 4], dtype=torch.int32, device="cuda")
+    got = torch.empty((4, n_out), device="cuda")
+    ops.mmq_run(blob, t, n_out, n_in, w.size + shift, 2, xm, bounds, None, 4, got, n_out)
+    one = host(ops.iq_mmvq(t, dev(w), ops.quantize_q8_1_rows(x), n_in, n_out, 4))
+    np.testing.assert_allclose(host(got)[:2], one[:2], rtol=1e-5, atol=1e-5 * np.abs(one).max())
+    np.testing.assert_allclose(host(got)[2:, ::-1], one[2:], rtol=1e-5, atol=1e-5 * np.abs(one).max())
+    # a group whose blob lies off a 4-byte boundary
+    L = ops.native_expert_layout(t, t, 256, 256)
+    e = np.concatenate([weights(t, 512, 256, 1).ravel(), weights(t, 256, 256, 2).ravel()])
+    assert e.size == L.down_off + 256 * L.d_row
+    eb = torch.zeros(e.size + shift + 16, dtype=torch.uint8, device="cuda")
+    eb[shift:shift + e.size] = dev(e)
+    xe = ops.quantize_q8_1_rows(x[:2, :256].contiguous())
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device="cuda")
+    scratch = torch.empty(ops.native_expert_scratch_bytes(2, 256), dtype=torch.uint8, device="cuda")
+    outs = []
+    for base in (dev(e), eb[shift:]):
+        out = torch.full((2, 256), float("nan"), device="cuda")
+        ops.native_expert_grouped(L, torch.tensor([base.data_ptr()], dtype=torch.int64, device="cuda"), i32(0, 2), i32(1),
+                                  i32(0, 1), i32(0, 1), 1, 2, xe, scratch, out)
+        outs.append(host(out))
+    assert np.array_equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("t", ALL)
 @pytest.mark.parametrize("x_every", [1, 3])
 def test_mmvq_ids(t, x_every):
     n_in, n_out, n_mat, count = 512, 80, 6, 11

@@ -300,20 +300,20 @@ __device__ __forceinline__ void unit_load(const uint8_t* row, int u, Unit& o, co
 }
 
 // ------------------------------------------------------------------ unit decode from global memory
-// unit_load reads a unit's fields as 16-bit words, which an LDS slab serves well and global memory does not: a Q4_K unit
-// is 22 load instructions of two bytes a lane.  Here the aligned 4-byte words around the fields are read in 16-byte
-// pieces and shifted into place: three load instructions for a Q4_K unit, three for Q8_0, eight for Q6_K.  Rows start on
-// 2-byte boundaries at least, as GGUF blocks of an even size do behind a 4-byte aligned matrix.  Only words that hold
-// bytes of the field are read.  Four dense products of 2048 x 6144 by four columns with their quantize launches: Q6_K
-// 55 -> 41 us, Q8_0 54 -> 40, Q4_K 46 -> 36; IQ3_S, its codebook in LDS (LdsTab), 51 -> 39.
+// The fields of a unit in global memory, which two-byte loads serve badly (22 of them for a Q4_K unit): the aligned 4-byte
+// words around the fields are read in 16-byte pieces and shifted into place: three load instructions for a Q4_K unit, three
+// for Q8_0, eight for Q6_K.  Only words that hold bytes of the field are read.  A GGUF matrix starts on a 4-byte boundary
+// and its rows on 2-byte ones; any other byte address (a byte stride of experts, an offset of the caller's) costs the same
+// shifts.  Four dense products of 2048 x 6144 by four columns with their quantize launches: Q6_K 55 -> 41 us, Q8_0 54 ->
+// 40, Q4_K 46 -> 36; IQ3_S, its codebook in LDS (LdsTab), 51 -> 39.
 typedef int v4i_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef int v2i_a4 __attribute__((ext_vector_type(2), aligned(4)));
 __device__ __forceinline__ uint32_t gld16(uintptr_t a) { return *(gbl_ptr<const uint16_t>) a; }
 __device__ __forceinline__ uint32_t gld8(uintptr_t a) { return *(gbl_ptr<const uint8_t>) a; }
-// 4 N bytes at a (2-byte aligned) as N words, N = 1, 2, 4 or 8.  shift (0 or 16) tells whether the bytes straddle words
+// 4 N bytes at a (any byte address) as N words, N = 1, 2, 4 or 8
 template <int N> __device__ __forceinline__ void gld_words(uintptr_t a, uint32_t (&w)[N]) {
     const uintptr_t b = a & ~(uintptr_t) 3;
-    const uint32_t sh = (uint32_t) (a & 2) * 8;
+    const uint32_t off = (uint32_t) a & 3u, sh = 8 * off;
     uint32_t r[N + 1];
     if constexpr (N >= 4) {
 #pragma unroll
@@ -330,7 +330,7 @@ template <int N> __device__ __forceinline__ void gld_words(uintptr_t a, uint32_t
         r[0] = *(gbl_ptr<const uint32_t>) b;
     }
     // the word after: read where the bytes straddle, else the last one again
-    r[N] = *(gbl_ptr<const uint32_t>) (b + 4 * (N - 1) + 2 * (a & 2));
+    r[N] = *(gbl_ptr<const uint32_t>) (b + 4 * (N - 1) + ((off + 3u) & 4u));
 #pragma unroll
     for (int k = 0; k < N; ++k) w[k] = __builtin_amdgcn_alignbit(r[k + 1], r[k], sh);
 }
