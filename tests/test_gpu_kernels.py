@@ -469,6 +469,57 @@ def test_mmq_run_few_rows(t, w_cols, w_rows, pad):
     assert (np.abs(got[:, :w_rows] - exp) <= 1e-5 * np.abs(exp) + 1e-5 * scale).all()
 
 
+def _cancelling_pair(t, w, cols):
+    """Two places of the first row's first unit whose weights have the same magnitude (Q4_K: the same code), and the sign
+    that makes w[i] - sign * w[j] zero: an activation unit (a at i, -sign a at j) whose dot product with the row is 0."""
+    v = O.dequantize(t, w[0], cols)[:32]
+    for i in range(32):
+        for j in range(i):
+            if v[i] != 0 and abs(v[i]) == abs(v[j]) and (t != Q4_K or v[i] == v[j]):
+                return i, j, float(np.sign(v[i] * v[j]))
+    raise AssertionError("no pair")
+
+
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("big,ratio", [(40.0, 18), (64.0, 20), (2.0 ** 8, 24), (2.0 ** 12, 30), (60000.0, 34), (16.0, 20)])
+@pytest.mark.parametrize("cols", [256, 768, 4352])
+def test_mmq_run_few_rows_wide_scales(t, big, ratio, cols):
+    """Activation units whose scales lie 2^18 to 2^34 apart within 256 values, the large unit's dot product with every row
+    exactly zero, so that the outputs are the small units' alone: within float32 rounding of the oracle's dot on the same
+    codes (a relative error of 1e-5 of the row's sum of magnitudes of the small units' terms).  One expert of 1 to 16
+    rows, all chunks in one window of activations or in several, one pass of output columns and two."""
+    rng = np.random.default_rng(t + ratio + cols)
+    w_rows, rows = 320, [1, 3, 16]
+    src = rng.normal(0, 0.02, (1, cols)).astype(np.float32)
+    src[0, 1] = src[0, 0]
+    base = ops.quantize_weights(t, src)
+    w = np.repeat(base, w_rows, axis=0)                 # the first block shared, the others each row's own
+    if cols > 256:
+        first = base.shape[1] // (cols // 256)
+        w[:, first:] = ops.quantize_weights(t, rng.normal(0, 0.02, (w_rows, cols)).astype(np.float32))[:, first:]
+    i, j, sign = _cancelling_pair(t, w, cols)
+    total, small = sum(rows), big * 2.0 ** -ratio
+    x = rng.normal(0, 127 * small / 3, (total, cols)).astype(np.float32)
+    x[:, :32] = 0.0
+    x[:, i], x[:, j] = 127 * big, -sign * 127 * big
+    bounds = np.concatenate([[0], np.cumsum(rows)]).astype(np.int32)
+    eb = (w.size + 255) // 256 * 256
+    blob = np.zeros((len(rows), eb), np.uint8)
+    blob[:, :w.size] = w.ravel()
+    print(f"few rows, wide scales t={t} big={big} 2^-{ratio} cols={cols}", flush=True)
+    xq = ops.mmq_quantize(dev(x), None, t, cols, cols, total)
+    dst = torch.full((total, w_rows), float("nan"), device="cuda")
+    ops.mmq_run(dev(blob.ravel()), t, w_rows, cols, eb, len(rows), xq, dev(bounds), None, total, dst, w_rows)
+    xb = O.quantize_q8_1(x)
+    d, _, q = O.q8_1_split(xb)
+    a = d.reshape(total, -1, 1).astype(np.float64) * q.reshape(total, -1, 32)
+    v = np.stack([O.dequantize(t, r, cols) for r in w]).astype(np.float64)
+    exp = a.reshape(total, cols)[:, 32:] @ v[:, 32:].T
+    mag = np.abs(a.reshape(total, cols)[:, 32:]) @ np.abs(v[:, 32:]).T
+    assert (a[:, 0] @ v[0, :32] == 0).all() and (mag > 0).all()
+    assert (np.abs(host(dst) - exp) <= 1e-5 * mag).all()
+
+
 @pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("N,FF,counts", [(512, 128, FEW_COUNTS), (2048, 384, FEW_COUNTS), (768, 256, [64]), (256, 128, [1])])
 def test_mmq_gate_up_swiglu_few_rows(t, N, FF, counts):

@@ -1031,8 +1031,11 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
 //   B = the activations with their scale, code * dx, as the sum of two fp16 numbers.  dx is an fp16 value, so the
 //       product has at most 18 bits: hi is the product rounded to a multiple of 2^e (dx in [2^e, 2^(e+1)): 8 bits), lo
 //       the rest (10 bits), both exact once dx has been multiplied by the power of two that puts the largest of the
-//       token's scales in the 256-value chunk in [16, 32) (exact while the chunk's scales lie within 2^18 of each
-//       other; a smaller one loses bits below 2^-40 of the chunk's largest product).
+//       token's scales in the 256-value chunk in [16, 32), as long as fp16 still holds the result: always where that
+//       largest scale is below 32 (scales are multiples of 2^-24, and then only grow), and down to 2^-18 of it where not.
+//       A block that meets a smaller scale goes over its chunks a second time with the units left out alone, 2^19 times
+//       larger: fp16 holds every one of those (below 2^-14 of a scale of at most 2^16).  A large unit that adds nothing to
+//       an output (zero weights, a sum of zero) therefore takes no bits from the small ones.
 // The sums over hi are integers of a common power of two that rarely need more than 24 bits, and lo has accumulators of
 // its own, so a chunk's sum is nearly exact in fp32; times the row's float scale and the token's power of two it is
 // added to the row's total (Q4_K's min term is a K = 8 product on the fp32 matrix cores).  Relative error against 64
@@ -1209,11 +1212,12 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
     int* const s_drow = reinterpret_cast<int*>(s_lds + L::DR);
     float* const s_dm = reinterpret_cast<float*>(s_lds + L::DM);
     uint64_t* const s_scan = reinterpret_cast<uint64_t*>(s_lds + L::SCAN);
-    int* const s_item = reinterpret_cast<int*>(s_scan + NW);  // expert, first row, rows
+    int* const s_item = reinterpret_cast<int*>(s_scan + NW);  // expert, first row, rows; whether a second round is needed
 
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int bx = (int) blockIdx.x % nbx;
+    if (tid == 0) s_item[3] = 0;
 
     // the codebook: this thread's grid entries, stored below
     constexpr int GE = small_grid<T>(), GPT = GE / NT;
@@ -1332,15 +1336,19 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
                 *(lds_ptr<v4i>) (s_lds + L::B + ptok[k] * tstride + 16 * (tid + NT * k - 16 * wch * ptok[k])) = q[k];
         if (tid < 2 * wch * nr) *(float4*) (s_dm + 8 * wch * stok8 + 4 * sp) = d;
     };
-    auto stage_f16 = [&](int v) {
+    // round 0: the units whose normalized scale fp16 holds; round 1: the others
+    auto stage_f16 = [&](int v, int round) {
         const int c = v * wch + sc;
         if (sc >= wch || c >= nchunks) return;
         const v4i bc = *(const v4i*) (aq + kChunk * c);
         const float4 x0 = *(const float4*) (ad + 8 * c), x1 = *(const float4*) (ad + 8 * c + 4);
         const float du = ad[8 * c + su];
         const float mx = fmaxf(fmaxf(fmaxf(x0.x, x0.y), fmaxf(x0.z, x0.w)), fmaxf(fmaxf(x1.x, x1.y), fmaxf(x1.z, x1.w)));
-        const int e = mx > 0.f ? __builtin_amdgcn_frexp_expf(mx) - 5 : 0;  // mx in [2^(e+4), 2^(e+5))
-        const float dn = __builtin_amdgcn_ldexpf(du, -e);
+        const int e = (mx > 0.f ? __builtin_amdgcn_frexp_expf(mx) - 5 : 0) - 19 * round;  // mx in [2^(e+4), 2^(e+5))
+        const float d0 = __builtin_amdgcn_ldexpf(du, -e - 19 * round);
+        const bool later = d0 < 1.f && (float) (_Float16) d0 != d0;  // (a NaN belongs to round 0)
+        if (later && round == 0) s_item[3] = 1;
+        const float dn = later == (round == 1) ? __builtin_amdgcn_ldexpf(du, -e) : 0.f;
         // 1.5 * 2^(10 + the scale's exponent): what a sum with it is rounded to is a multiple of that power of two
         const float mg = dn > 0.f ? __builtin_amdgcn_ldexpf(1.5f, __builtin_amdgcn_frexp_expf(dn) + 9) : 0.f;
         const _Float16 dh = (_Float16) dn, mh = (_Float16) mg;
@@ -1364,15 +1372,20 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
         }
         if (su == 0 && sh == 0) s_ex[sc * nr + stok] = e;
         if constexpr (Q4K) {
-            if (sh == 0) s_dm[(sc * 8 + su) * nr + stok] = du * (float) am[8 * c + su];
+            if (sh == 0) s_dm[(sc * 8 + su) * nr + stok] = round == 0 ? du * (float) am[8 * c + su] : 0.f;
         }
     };
-    auto stage_b = [&](int v) {
+    int sv = 0, sr = 0;   // the window in LDS and its round
+    bool again = false;  // some unit is left for round 1 (the same in every thread once every window has been staged)
+    auto stage_b = [&](int v, int round) {
         if constexpr (Q80) stage_q80(v);
-        else stage_f16(v);
+        else stage_f16(v, round);
+        __syncthreads();
+        if constexpr (!Q80) again = __builtin_amdgcn_readfirstlane(s_item[3]) != 0;
+        sv = v;
+        sr = round;
     };
-    stage_b(0);
-    __syncthreads();
+    stage_b(0, 0);
 
     const v4f zero = {0.f, 0.f, 0.f, 0.f};
     const int tokc = min(lr, nr - 1);  // this lane's token, a row past the last taking the last
@@ -1383,99 +1396,106 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
 #pragma unroll
             for (int s = 0; s < kSTok / 4; ++s) part[s][0] = part[s][1] = zero;
         }
-        int cw = 0;  // the chunk's place in its window
-        for (int c = 0; c < nchunks; ++c, ++cw) {
-            if (nwin > 1 && (cw == wch || (c == 0 && p > 0))) {  // the next window
+        for (int round = 0;; ++round) {
+            if (sv != 0 || sr != round) {  // the first window again
                 __syncthreads();
-                stage_b(cw == wch ? c / wch : 0);
-                __syncthreads();
-                cw = 0;
+                stage_b(0, round);
             }
-            // this iteration's weights; the next one's requested (the last one's again after the last)
-            MmqRaw<T> W[2] = {R[0], R[1]};
-            const int sft = Q4K ? 0 : (int) (((uint32_t) row_base(p, c, 0) + lro + 2) & 2) * 8;
-            {
-                const int np = c + 1 < nchunks ? p : min(p + 1, npass - 1);
-                const int nc = c + 1 < nchunks ? c + 1 : p + 1 < npass ? 0 : c;
-                fetch_w(R, np, nc);
-            }
-            if constexpr (Q80) {
-                const int ci = lr >> 2;  // the lane group whose units this lane's column holds
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    s_uw[wave][2 * g][16 * t + lr] = h2f((uint16_t) W[t].q[0][0]);
-                    s_uw[wave][2 * g + 1][16 * t + lr] = h2f((uint16_t) ((uint32_t) W[t].q[2][0] >> 16));
+            int cw = 0;  // the chunk's place in its window
+            for (int c = 0; c < nchunks; ++c, ++cw) {
+                if (nwin > 1 && cw == wch) {  // the next window
+                    __syncthreads();
+                    stage_b(sv + 1, round);
+                    cw = 0;
                 }
-                wave_lds_order();
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    auto word = [&](int k) { return k == 16 ? W[t].q4 : W[t].q[(k >> 2) & 3][k & 3]; };
-                    v4i A[2][2];  // [unit][half]
-                    v4f dw[2];
-#pragma unroll
-                    for (int k = 0; k < 8; ++k) {
-                        A[0][k >> 2][k & 3] = (int) __builtin_amdgcn_alignbit((uint32_t) word(k + 1), (uint32_t) word(k), 16);
-                        A[1][k >> 2][k & 3] = word(9 + k);
-                    }
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) dw[j] = *(lds_ptr<const v4f>) &s_uw[wave][2 * ci + j][16 * t + 4 * g];
-#pragma unroll
-                    for (int s = 0; s < kSTok / 4; ++s) {
-                        if (4 * s >= nr) break;  // the same in every lane
-                        const int tok = min(4 * s + (lr & 3), nr - 1);
-                        const uint8_t* const b = s_lds + (ci == g ? L::B + tok * tstride + 256 * cw + 64 * g : L::EX);
-#pragma unroll
-                        for (int j = 0; j < 2; ++j) {
-                            const v4i b0 = *(lds_ptr<const v4i>) (b + 32 * j), b1 = *(lds_ptr<const v4i>) (b + 32 * j + 16);
-                            const float dx = s_dm[8 * wch * tok + 8 * cw + 2 * ci + j];
-                            v4i C = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[j][0], b0, v4i{0, 0, 0, 0}, 0, 0, 0);
-                            C = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[j][1], b1, C, 0, 0, 0);
-#pragma unroll
-                            for (int i = 0; i < 4; ++i)
-                                part[s][t][i] = __builtin_fmaf((float) C[i], dw[j][i] * dx, part[s][t][i]);
-                        }
-                    }
+                // this iteration's weights; the next one's requested (the last one's again after the last)
+                MmqRaw<T> W[2] = {R[0], R[1]};
+                const int sft = Q4K ? 0 : (int) (((uint32_t) row_base(p, c, 0) + lro + 2) & 2) * 8;
+                {
+                    const bool same = c + 1 < nchunks || (round == 0 && again);
+                    const int np = same ? p : min(p + 1, npass - 1);
+                    const int nc = c + 1 < nchunks ? c + 1 : same || p + 1 < npass ? 0 : c;
+                    fetch_w(R, np, nc);
                 }
-                wave_lds_order();  // the next chunk's scales go to the same place
-            } else {
-                MmqScale<T> S[2];
-#pragma unroll
-                for (int t = 0; t < 2; ++t) raw_scales<T>(W[t], sft, g, S[t]);
-                if (g < 2) s_dw[wave][lane & 31] = g == 0 ? S[0].d : S[1].d;
-                v4f hi[2], lo[2];
-                const uint8_t* const bw = s_lds + L::B + (cw * 8 * 8 + g) * nr * 16 + tokc * 16;
-#pragma unroll
-                for (int s = 0; s < 8; ++s) {
-                    v4i A[2];
-#pragma unroll
-                    for (int t = 0; t < 2; ++t) A[t] = raw_frag<T>(W[t], S[t], sft, s, s_lds + L::TAB);
-                    const v4i bh = *(lds_ptr<const v4i>) (bw + (s * 8) * nr * 16);
-                    const v4i bl = *(lds_ptr<const v4i>) (bw + (s * 8 + 4) * nr * 16);
+                if constexpr (Q80) {
+                    const int ci = lr >> 2;  // the lane group whose units this lane's column holds
 #pragma unroll
                     for (int t = 0; t < 2; ++t) {
-                        hi[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t]), __builtin_bit_cast(v8h, bh),
-                                                                       s == 0 ? zero : hi[t], 0, 0, 0);
-                        lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t]), __builtin_bit_cast(v8h, bl),
-                                                                       s == 0 ? zero : lo[t], 0, 0, 0);
+                        s_uw[wave][2 * g][16 * t + lr] = h2f((uint16_t) W[t].q[0][0]);
+                        s_uw[wave][2 * g + 1][16 * t + lr] = h2f((uint16_t) ((uint32_t) W[t].q[2][0] >> 16));
                     }
-                }
-                if constexpr (Q4K) {
+                    wave_lds_order();
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const float bm = s_dm[(cw * 8 + 2 * g + h) * nr + tokc];
+                    for (int t = 0; t < 2; ++t) {
+                        auto word = [&](int k) { return k == 16 ? W[t].q4 : W[t].q[(k >> 2) & 3][k & 3]; };
+                        v4i A[2][2];  // [unit][half]
+                        v4f dw[2];
 #pragma unroll
-                        for (int t = 0; t < 2; ++t)
-                            tot[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[t].mn[h], bm, tot[t], 0, 0, 0);
+                        for (int k = 0; k < 8; ++k) {
+                            A[0][k >> 2][k & 3] = (int) __builtin_amdgcn_alignbit((uint32_t) word(k + 1), (uint32_t) word(k), 16);
+                            A[1][k >> 2][k & 3] = word(9 + k);
+                        }
+#pragma unroll
+                        for (int j = 0; j < 2; ++j) dw[j] = *(lds_ptr<const v4f>) &s_uw[wave][2 * ci + j][16 * t + 4 * g];
+#pragma unroll
+                        for (int s = 0; s < kSTok / 4; ++s) {
+                            if (4 * s >= nr) break;  // the same in every lane
+                            const int tok = min(4 * s + (lr & 3), nr - 1);
+                            const uint8_t* const b = s_lds + (ci == g ? L::B + tok * tstride + 256 * cw + 64 * g : L::EX);
+#pragma unroll
+                            for (int j = 0; j < 2; ++j) {
+                                const v4i b0 = *(lds_ptr<const v4i>) (b + 32 * j), b1 = *(lds_ptr<const v4i>) (b + 32 * j + 16);
+                                const float dx = s_dm[8 * wch * tok + 8 * cw + 2 * ci + j];
+                                v4i C = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[j][0], b0, v4i{0, 0, 0, 0}, 0, 0, 0);
+                                C = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[j][1], b1, C, 0, 0, 0);
+#pragma unroll
+                                for (int i = 0; i < 4; ++i)
+                                    part[s][t][i] = __builtin_fmaf((float) C[i], dw[j][i] * dx, part[s][t][i]);
+                            }
+                        }
                     }
-                }
-                const float dt = __builtin_amdgcn_ldexpf(1.0f, s_ex[cw * nr + tokc]);
+                    wave_lds_order();  // the next chunk's scales go to the same place
+                } else {
+                    MmqScale<T> S[2];
 #pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    const v4f dw = *(lds_ptr<const v4f>) &s_dw[wave][16 * t + 4 * g];
+                    for (int t = 0; t < 2; ++t) raw_scales<T>(W[t], sft, g, S[t]);
+                    if (g < 2) s_dw[wave][lane & 31] = g == 0 ? S[0].d : S[1].d;
+                    v4f hi[2], lo[2];
+                    const uint8_t* const bw = s_lds + L::B + (cw * 8 * 8 + g) * nr * 16 + tokc * 16;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) tot[t][i] = __builtin_fmaf(hi[t][i] + lo[t][i], dw[i] * dt, tot[t][i]);
+                    for (int s = 0; s < 8; ++s) {
+                        v4i A[2];
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) A[t] = raw_frag<T>(W[t], S[t], sft, s, s_lds + L::TAB);
+                        const v4i bh = *(lds_ptr<const v4i>) (bw + (s * 8) * nr * 16);
+                        const v4i bl = *(lds_ptr<const v4i>) (bw + (s * 8 + 4) * nr * 16);
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) {
+                            hi[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t]), __builtin_bit_cast(v8h, bh),
+                                                                           s == 0 ? zero : hi[t], 0, 0, 0);
+                            lo[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, A[t]), __builtin_bit_cast(v8h, bl),
+                                                                           s == 0 ? zero : lo[t], 0, 0, 0);
+                        }
+                    }
+                    if constexpr (Q4K) {
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const float bm = s_dm[(cw * 8 + 2 * g + h) * nr + tokc];
+#pragma unroll
+                            for (int t = 0; t < 2; ++t)
+                                tot[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(S[t].mn[h], bm, tot[t], 0, 0, 0);
+                        }
+                    }
+                    const float dt = __builtin_amdgcn_ldexpf(1.0f, s_ex[cw * nr + tokc]);
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) {
+                        const v4f dw = *(lds_ptr<const v4f>) &s_dw[wave][16 * t + 4 * g];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) tot[t][i] = __builtin_fmaf(hi[t][i] + lo[t][i], dw[i] * dt, tot[t][i]);
+                    }
                 }
             }
+            if (Q80 || round == 1 || !again) break;
         }
         if constexpr (Q80) {
             // the token's four columns, 4 apart, then set lr / 4's sums: token lr, the same lane for every row
