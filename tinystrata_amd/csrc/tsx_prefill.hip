@@ -356,6 +356,9 @@ template <typename T> __device__ __forceinline__ lds_ptr<const T> lds_base(const
     return (lds_ptr<const T>) (uintptr_t) a;
 }
 __device__ __forceinline__ void wave_lds_order() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// the same for the compiler alone: a wave's LDS instructions run in their order, so lanes of one wave that hand each other
+// values through LDS need only that the compiler keeps the stores before the loads (and these before the next stores)
+__device__ __forceinline__ void wave_lds_sequence() { asm volatile("" ::: "memory"); }
 
 // exclusive prefix sum over the NT threads of the block (v per thread), and the total
 template <int NT, typename V>
@@ -1460,6 +1463,7 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
 #pragma unroll
                     for (int t = 0; t < 2; ++t) raw_scales<T>(W[t], sft, g, S[t]);
                     if (g < 2) s_dw[wave][lane & 31] = g == 0 ? S[0].d : S[1].d;
+                    wave_lds_sequence();
                     v4f hi[2], lo[2];
                     const uint8_t* const bw = s_lds + L::B + (cw * 8 * 8 + g) * nr * 16 + tokc * 16;
 #pragma unroll
@@ -1493,6 +1497,7 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
 #pragma unroll
                         for (int i = 0; i < 4; ++i) tot[t][i] = __builtin_fmaf(hi[t][i] + lo[t][i], dw[i] * dt, tot[t][i]);
                     }
+                    wave_lds_sequence();  // the next chunk's scales go to the same place
                 }
             }
             if (Q80 || round == 1 || !again) break;
