@@ -245,6 +245,25 @@ def test_mmq_quantize_route_matches_the_two_calls(rows, E, k):
     assert (host(wts).view(np.int32) == host(wts_s).view(np.int32)).all()
 
 
+@pytest.mark.parametrize("shared,n,k", [(False, 2048, 8), (True, 1568, 3), (True, 96, 1), (False, 16384, 4)])
+def test_combine_norm_forms_agree(shared, n, k):
+    """Rows on 16-byte boundaries (four columns per thread) and one float off them (one): the same x, h and hq bits."""
+    g = torch.Generator(device="cuda").manual_seed(n)
+    rand = lambda *s: torch.randn(s, generator=g, device="cuda")
+    T = 5
+    x, parts, wts, wn = rand(T, n), rand(T * k, n), rand(T, k), rand(n)
+    sh, sg = (rand(T, n), rand(T)) if shared else (None, None)
+    outs = []
+    for pad in (0, 1):
+        xd = x.clone()
+        h = torch.full((T * n + pad,), float("nan"), device="cuda")[pad:].view(T, n)
+        hq = torch.zeros((T, n // 32 * 36), dtype=torch.uint8, device="cuda")
+        ops.moe_combine_norm(xd, parts, wts, k, wn, 1e-6, h, hq, shared=sh, sgate=sg)
+        outs.append((host(xd), host(h), host(hq)))
+    for a, b in zip(*outs):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+
+
 @pytest.mark.parametrize("shared,prow,n", [(False, False, 2048), (True, True, 2048), (True, False, 4096),
                                            (False, True, 96)])
 @pytest.mark.parametrize("pad,k", [(0, 8), (0, 3), (1, 8)])   # rows 16-byte aligned (four columns per thread), and not

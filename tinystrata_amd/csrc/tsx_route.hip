@@ -328,7 +328,8 @@ __global__ void __launch_bounds__(kNormThreads) combine_norm_kernel(float* __res
 }
 
 // the same, four columns per thread (every row 16-byte aligned): a token's k part rows, the shared row and x requested
-// together as 16-byte loads, and the norm's half four columns a lane, eight lanes a Q8_1 block.  The scalar form above
+// together as 16-byte loads, and the norm's half four columns a lane, eight lanes a Q8_1 block.  The sum of squares is
+// taken from the row in LDS in the scalar form's order, so that x, h and hq are that form's bit for bit.  The scalar form
 // waits for its part rows' 4-byte loads one column at a time: 777 tokens x 2048, top-8: 32 -> 14 us with the launch gap
 // (the parts come from the memory-side cache)
 __device__ __forceinline__ float lane_xor4(float v) { return __shfl_xor(v, 4, 8); }
@@ -349,7 +350,6 @@ __global__ void __launch_bounds__(kNormThreads) combine_norm4_kernel(float* __re
     auto part = [&](int j, int i) {
         return *(const float4*) (parts + (int64_t) (prow ? prow[t * k + j] : t * k + j) * n + i);
     };
-    float q = 0.f;
     for (int i = 4 * tid; i < n; i += 4 * kNormThreads) {
         const float4 xv = *(const float4*) (xr + i);
         float4 p = part(0, i);
@@ -375,12 +375,11 @@ __global__ void __launch_bounds__(kNormThreads) combine_norm4_kernel(float* __re
         const float4 v = {xv.x + acc.x, xv.y + acc.y, xv.z + acc.z, xv.w + acc.w};
         *(float4*) (xr + i) = v;
         *(float4*) (s_row + i) = v;
-        q += v.x * v.x;
-        q += v.y * v.y;
-        q += v.z * v.z;
-        q += v.w * v.w;
     }
-    q = reduce64(q, OpAddF());
+    __syncthreads();
+    float q = 0.f;
+    for (int i = tid; i < n; i += kNormThreads) q += s_row[i] * s_row[i];
+    q = tree_sum<64>(q);
     if ((tid & 63) == 0) s_red[tid >> 6] = q;
     __syncthreads();
     float sum = 0.f;
