@@ -269,7 +269,9 @@ TSX_API int tsx_moe_mmq_gate_up_swiglu(const void* w, int type, int64_t n_ff, in
 
 /* ------------------------------------------------------------------------------------------------ checks and data */
 /* The integer contract: sums[(r*ncols + c)*nsub + u] = sum over sub-block u (32 values) of w_int * a_int, and
- * qsums (may be null) the same for sum a_int, for rows [0, n_rows) of W against ncols Q8_1 activations.
+ * qsums (may be null) the same for sum a_int, for rows [0, n_rows) of W against ncols Q8_1 activations.  An expert
+ * format (IQ3_XXS, IQ3_S, Q4_K, Q8_0) on a 16-byte boundary is decoded as the fused decode layer does it, from LDS; off
+ * that boundary, and Q4_0 and Q6_K, as the kernel-by-kernel products do, from global memory.
  * No reference counterpart: the tests compare these to the oracle bit for bit. */
 TSX_API int tsx_moe_subblock_sums(int type, const void* w, int64_t n_in, int64_t n_rows, const void* x_q8_1,
                                   int64_t ncols, int32_t* sums, int32_t* qsums, void* stream);

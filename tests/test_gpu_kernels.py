@@ -103,6 +103,23 @@ def test_subblock_sums_random_bytes_exact():
 
 
 @pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("n,rows", [(256, 1), (768, 11), (2048, 61)])
+@pytest.mark.parametrize("shift", [0, 4])
+def test_subblock_sums_both_decoders_random_bytes(t, n, rows, shift):
+    """Both unit decoders, the fused decode layer's (rows on a 16-byte boundary, read from LDS) and the kernel-by-kernel
+    products' (off it, read from global memory), over random block bytes: every code, index and sign;
+    rows that start at every even offset of a 16-byte piece, a last block of few units, exact."""
+    rng = np.random.default_rng(n + t)
+    w = rng.integers(0, 256, (rows, O.row_bytes(t, n)), dtype=np.uint8)
+    buf = torch.zeros(w.size + 16, dtype=torch.uint8, device="cuda")
+    buf[shift:shift + w.size] = dev(w.ravel())
+    xq = O.quantize_q8_1(rng.normal(0, 1, (2, n)).astype(np.float32))
+    s, q = ops.subblock_sums(t, buf[shift:], n, rows, dev(xq), 2)
+    es, eq = O.subblock_sums(t, w, n, rows, xq, 2)
+    assert (host(s) == es).all() and (host(q) == eq).all()
+
+
+@pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("n_in,n_out,ncols", [(2048, 96, 1), (2048, 40, 4), (512, 2048, 8), (768, 64, 3)])
 def test_mmvq(t, n_in, n_out, ncols):
     if n_in % O.BLOCK[t][0]:

@@ -282,18 +282,40 @@ __global__ void __launch_bounds__(kThreads) mmvq_many_kernel(Src src, uint64_t r
             if (r0 + RPW * j < n_out) yj[r0 + RPW * j] = acc[j][0];
 }
 
-// the integer contract, one thread per (row, unit)
-template <int T>
+// the integer contract, one thread per (row, unit).  Two decoders read units, one from global memory (this file's products,
+// the prompt's row-dot product) and one from LDS (the fused decode layer): LDS takes the latter, for which a block's
+// consecutive units lie in LDS as one row, with the layer's copies of the codebook
+template <int T, bool LDS>
 __global__ void __launch_bounds__(kThreads) subblock_sums_kernel(const uint8_t* __restrict__ w, uint64_t row_bytes,
                                                                  int nu, int64_t n_rows,
                                                                  const tsx_block_q8_1* __restrict__ x, int64_t ncols,
                                                                  int32_t* __restrict__ sums, int32_t* __restrict__ qsums) {
     const int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n_rows * nu) return;
-    const int64_t r = i / nu;
+    const int64_t r = min(i / nu, n_rows - 1);
     const int u = (int) (i % nu);
     Unit wu;
-    unit_load_global<T>(w + (uint64_t) r * row_bytes, u, wu, grid_const());
+    if constexpr (LDS) {
+        constexpr int CB = kThreads / Fmt<T>::upb * Fmt<T>::bytes, REP = rep_lds_bytes<T>();  // CB: a multiple of 16
+        __shared__ __attribute__((aligned(16))) uint8_t s_w[CB + 16];  // (a Q8_0 unit's words end up to 2 bytes behind it)
+        __shared__ __attribute__((aligned(16))) uint8_t s_rep[REP > 0 ? REP : 16];
+        const int64_t base = (int64_t) blockIdx.x * CB, left = n_rows * (int64_t) row_bytes - base;
+        const int nb = (int) min(left, (int64_t) CB);
+        for (int k = threadIdx.x; k < nb / 16; k += kThreads) ((v4i*) s_w)[k] = ((const v4i*) (w + base))[k];
+        if ((int) threadIdx.x < nb % 16) s_w[nb / 16 * 16 + threadIdx.x] = w[base + nb / 16 * 16 + threadIdx.x];
+        if constexpr (REP > 0) {
+            uint64_t v[(rep_stores<T>() + kThreads - 1) / kThreads];
+            rep_fetch<T>(v, (int) threadIdx.x, kThreads);
+            const RepTab<T> tab = rep_store<T>(s_rep, v, (int) threadIdx.x, kThreads);
+            __syncthreads();
+            if (i < n_rows * nu) unit_load<T>(s_w, (int) threadIdx.x, wu, tab);
+        } else {
+            __syncthreads();
+            if (i < n_rows * nu) unit_load<T>(s_w, (int) threadIdx.x, wu, grid_const());
+        }
+    } else {
+        unit_load_global<T>(w + (uint64_t) r * row_bytes, u, wu, grid_const());
+    }
+    if (i >= n_rows * nu) return;
     for (int64_t c = 0; c < ncols; ++c) {
         Act a;
         act_load(x + c * nu + u, a);
@@ -514,11 +536,16 @@ TSX_API int tsx_moe_subblock_sums(int type, const void* w, int64_t n_in, int64_t
                 "tsx_moe_subblock_sums: w, x, sums");
     const int nu = (int) (n_in / 32);
     if (n_rows == 0) return TSX_OK;
-    return with_mmvq_type(type, [&](auto T) {
-        subblock_sums_kernel<decltype(T)::value><<<blocks_for(n_rows * nu, kThreads), kThreads, 0, (hipStream_t) stream>>>(
-            (const uint8_t*) w, rb, nu, n_rows, (const tsx_block_q8_1*) x_q8_1, ncols, sums, qsums);
+    const auto launch = [&](auto T, auto lds) {
+        subblock_sums_kernel<decltype(T)::value, decltype(lds)::value>
+            <<<blocks_for(n_rows * nu, kThreads), kThreads, 0, (hipStream_t) stream>>>(
+                (const uint8_t*) w, rb, nu, n_rows, (const tsx_block_q8_1*) x_q8_1, ncols, sums, qsums);
         return launch_status("tsx_moe_subblock_sums");
-    });
+    };
+    // an expert format on the decode layer's boundary by that layer's decoder
+    if (aligned(w, 16) && tsx_weight_type_ok(type))
+        return with_type(type, [&](auto T) { return launch(T, std::integral_constant<bool, true>{}); });
+    return with_mmvq_type(type, [&](auto T) { return launch(T, std::integral_constant<bool, false>{}); });
 }
 
 }  // extern "C"
