@@ -51,8 +51,9 @@ __global__ void __launch_bounds__(kThreads) swiglu_entries_kernel(const float* _
 
 // ------------------------------------------------------------------ row dots
 // acc[j][c] = rows[j] . x[c] for c < n, the R rows' LPR lanes each taking units l, l + LPR, ...; reduced over the LPR
-// lanes.  A unit's activations (36 bytes a column, against 18 of Q4_K weights) are read once for the R rows
-template <int T, int LPR, int NC, int R>
+// lanes.  A unit's activations (36 bytes a column, against 18 of Q4_K weights) are read once for the R rows.  BYTES: the rows
+// start on odd addresses
+template <int T, int LPR, int NC, int R, bool BYTES>
 __device__ __forceinline__ void row_dots(const uint8_t* const (&rows)[R], const tsx_block_q8_1* const (&xs)[NC], int n,
                                          int nu, int l, const LdsTab<T>& tab, float (&acc)[R][NC]) {
 #pragma unroll
@@ -62,7 +63,7 @@ __device__ __forceinline__ void row_dots(const uint8_t* const (&rows)[R], const 
     for (int u = l; u < nu; u += LPR) {
         Unit w[R];
 #pragma unroll
-        for (int j = 0; j < R; ++j) unit_load_global<T>(rows[j], u, w[j], tab);
+        for (int j = 0; j < R; ++j) unit_load_global<T, BYTES>(rows[j], u, w[j], tab);
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
             if (c < n) {
@@ -91,6 +92,18 @@ inline int rows_per_lane_group(int64_t rows, int lpr) {
     const int64_t waves = rows / (kWave / lpr);
     return waves >= 4 * kRowsPerWaveMin ? 4 : waves >= 2 * kRowsPerWaveMin ? 2 : 1;
 }
+// f(rows at once, whether they start on odd addresses, first row) over a wave's R rows RPW apart.  A matrix that starts on an
+// odd address (a byte stride or offset of the caller's; every row then does) is read row by row, in a loop of its own
+// beside the others', whose code it leaves as it is
+template <int R, int RPW, typename F>
+__device__ __forceinline__ void rows_of_wave(const uint8_t* matrix, int row0, F&& f) {
+    if (__builtin_expect((uintptr_t) matrix & 1, 0)) {
+#pragma unroll 1
+        for (int j = 0; j < R; ++j) f(std::integral_constant<int, 1>{}, std::true_type{}, row0 + RPW * j);
+    } else {
+        f(std::integral_constant<int, R>{}, std::false_type{}, row0);
+    }
+}
 template <typename F>
 int with_rows(int r, F&& f) {
     switch (r) {
@@ -115,38 +128,39 @@ __global__ void __launch_bounds__(kThreads) expert_gu_kernel(const uint64_t* __r
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
     const int FF = (int) L.n_ff, nu = (int) (L.n_embd / 32);
-    const int row0 = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
-    uint64_t off[R];
-    float* dst[R];
-#pragma unroll
-    for (int j = 0; j < R; ++j) {  // a row past the last repeats the last and stores nothing
-        const int row = min(row0 + RPW * j, 2 * FF - 1);
-        const bool is_up = row >= FF;
-        const int r = is_up ? row - FF : row;
-        off[j] = (is_up ? L.up_off : 0) + (uint64_t) r * L.gu_row;
-        dst[j] = (is_up ? up : gate) + r;
-    }
+    const int first = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
     const int ng = *n_groups;
     for (int g = blockIdx.y; g < ng; g += gridDim.y) {
-        const uint8_t* wr[R];
-#pragma unroll
-        for (int j = 0; j < R; ++j) wr[j] = (const uint8_t*) grp_ptr[g] + off[j];
+        const uint8_t* const blob = (const uint8_t*) grp_ptr[g];
         const int e0 = grp_start[g], e1 = grp_start[g + 1];
-        for (int e = e0; e < e1; e += kNC) {
-            const int n = min(kNC, e1 - e);
-            const tsx_block_q8_1* xs[kNC];
+        rows_of_wave<R, RPW>(blob, first, [&](auto at_once, auto bytes, int row0) {
+            constexpr int RR = decltype(at_once)::value;
+            const uint8_t* wr[RR];
+            float* dst[RR];
 #pragma unroll
-            for (int c = 0; c < kNC; ++c) xs[c] = xq + (int64_t) ent_tok[e + min(c, n - 1)] * nu;
-            float acc[R][kNC];
-            row_dots<T, LPR, kNC, R>(wr, xs, n, nu, l, tab, acc);
-            if (l == 0)
+            for (int j = 0; j < RR; ++j) {  // a row past the last repeats the last and stores nothing
+                const int row = min(row0 + RPW * j, 2 * FF - 1);
+                const bool is_up = row >= FF;
+                const int r = is_up ? row - FF : row;
+                wr[j] = blob + (is_up ? L.up_off : 0) + (uint64_t) r * L.gu_row;
+                dst[j] = (is_up ? up : gate) + r;
+            }
+            for (int e = e0; e < e1; e += kNC) {
+                const int n = min(kNC, e1 - e);
+                const tsx_block_q8_1* xs[kNC];
 #pragma unroll
-                for (int j = 0; j < R; ++j)
-                    if (row0 + RPW * j < 2 * FF)
+                for (int c = 0; c < kNC; ++c) xs[c] = xq + (int64_t) ent_tok[e + min(c, n - 1)] * nu;
+                float acc[RR][kNC];
+                row_dots<T, LPR, kNC, RR, decltype(bytes)::value>(wr, xs, n, nu, l, tab, acc);
+                if (l == 0)
 #pragma unroll
-                        for (int c = 0; c < kNC; ++c)
-                            if (c < n) dst[j][(int64_t) (e + c) * FF] = acc[j][c];
-        }
+                    for (int j = 0; j < RR; ++j)
+                        if (row0 + RPW * j < 2 * FF)
+#pragma unroll
+                            for (int c = 0; c < kNC; ++c)
+                                if (c < n) dst[j][(int64_t) (e + c) * FF] = acc[j][c];
+            }
+        });
     }
 }
 
@@ -165,29 +179,32 @@ __global__ void __launch_bounds__(kThreads) expert_down_kernel(const uint64_t* _
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
     const int N = (int) L.n_embd, nu = (int) (L.n_ff / 32);
-    const int r0 = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
+    const int first = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
     const int ng = *n_groups;
     for (int g = blockIdx.y; g < ng; g += gridDim.y) {
-        const uint8_t* wr[R];
-#pragma unroll
-        for (int j = 0; j < R; ++j)
-            wr[j] = (const uint8_t*) grp_ptr[g] + L.down_off + (uint64_t) min(r0 + RPW * j, N - 1) * L.d_row;
+        const uint8_t* const blob = (const uint8_t*) grp_ptr[g];
         const int e0 = grp_start[g], e1 = grp_start[g + 1];
-        for (int e = e0; e < e1; e += kNC) {
-            const int n = min(kNC, e1 - e);
-            const tsx_block_q8_1* xs[kNC];
+        rows_of_wave<R, RPW>(blob, first, [&](auto at_once, auto bytes, int r0) {
+            constexpr int RR = decltype(at_once)::value;
+            const uint8_t* wr[RR];
 #pragma unroll
-            for (int c = 0; c < kNC; ++c) xs[c] = hq + (int64_t) (e + min(c, n - 1)) * nu;
-            float acc[R][kNC];
-            row_dots<T, LPR, kNC, R>(wr, xs, n, nu, l, tab, acc);
-            if (l == 0)
+            for (int j = 0; j < RR; ++j) wr[j] = blob + L.down_off + (uint64_t) min(r0 + RPW * j, N - 1) * L.d_row;
+            for (int e = e0; e < e1; e += kNC) {
+                const int n = min(kNC, e1 - e);
+                const tsx_block_q8_1* xs[kNC];
 #pragma unroll
-                for (int j = 0; j < R; ++j)
-                    if (r0 + RPW * j < N)
+                for (int c = 0; c < kNC; ++c) xs[c] = hq + (int64_t) (e + min(c, n - 1)) * nu;
+                float acc[RR][kNC];
+                row_dots<T, LPR, kNC, RR, decltype(bytes)::value>(wr, xs, n, nu, l, tab, acc);
+                if (l == 0)
 #pragma unroll
-                        for (int c = 0; c < kNC; ++c)
-                            if (c < n) out[(int64_t) ent_dst[e + c] * N + r0 + RPW * j] = acc[j][c];
-        }
+                    for (int j = 0; j < RR; ++j)
+                        if (r0 + RPW * j < N)
+#pragma unroll
+                            for (int c = 0; c < kNC; ++c)
+                                if (c < n) out[(int64_t) ent_dst[e + c] * N + r0 + RPW * j] = acc[j][c];
+            }
+        });
     }
 }
 
@@ -203,25 +220,28 @@ __global__ void __launch_bounds__(kThreads) mmvq_kernel(const uint8_t* __restric
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
     const int nu = n_in / 32;
-    const int r0 = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
-    const uint8_t* wr[R];
+    const int first = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
+    rows_of_wave<R, RPW>(w, first, [&](auto at_once, auto bytes, int r0) {
+        constexpr int RR = decltype(at_once)::value;
+        const uint8_t* wr[RR];
 #pragma unroll
-    for (int j = 0; j < R; ++j) wr[j] = w + (uint64_t) min(r0 + RPW * j, n_out - 1) * row_bytes;
-    for (int c0 = 0; c0 < ncols; c0 += kNC) {
-        const int n = min(kNC, ncols - c0);
-        const tsx_block_q8_1* xs[kNC];
+        for (int j = 0; j < RR; ++j) wr[j] = w + (uint64_t) min(r0 + RPW * j, n_out - 1) * row_bytes;
+        for (int c0 = 0; c0 < ncols; c0 += kNC) {
+            const int n = min(kNC, ncols - c0);
+            const tsx_block_q8_1* xs[kNC];
 #pragma unroll
-        for (int c = 0; c < kNC; ++c) xs[c] = x + (int64_t) (c0 + min(c, n - 1)) * nu;
-        float acc[R][kNC];
-        row_dots<T, LPR, kNC, R>(wr, xs, n, nu, l, tab, acc);
-        if (l == 0)
+            for (int c = 0; c < kNC; ++c) xs[c] = x + (int64_t) (c0 + min(c, n - 1)) * nu;
+            float acc[RR][kNC];
+            row_dots<T, LPR, kNC, RR, decltype(bytes)::value>(wr, xs, n, nu, l, tab, acc);
+            if (l == 0)
 #pragma unroll
-            for (int j = 0; j < R; ++j)
-                if (r0 + RPW * j < n_out)
+                for (int j = 0; j < RR; ++j)
+                    if (r0 + RPW * j < n_out)
 #pragma unroll
-                    for (int c = 0; c < kNC; ++c)
-                        if (c < n) y[(int64_t) (c0 + c) * n_out + r0 + RPW * j] = acc[j][c];
-    }
+                        for (int c = 0; c < kNC; ++c)
+                            if (c < n) y[(int64_t) (c0 + c) * n_out + r0 + RPW * j] = acc[j][c];
+        }
+    });
 }
 
 // Several matrices of one format and shape (blockIdx.y = matrix j), one activation column each: y_j[r] = W_j[r] . x_j.
@@ -264,22 +284,26 @@ __global__ void __launch_bounds__(kThreads) mmvq_many_kernel(Src src, uint64_t r
     constexpr int RPW = kWave / LPR;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
-    const int r0 = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
+    const int first = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
     const uint8_t* w = nullptr;
     const tsx_block_q8_1* xj = nullptr;
     float* yj = nullptr;
-    float acc[R][1] = {};
-    if (src.at((int) blockIdx.y, w, xj, yj)) {  // else an id outside the table: the matrix's outputs are zero
-        const tsx_block_q8_1* xs[1] = {xj};
-        const uint8_t* wr[R];
+    const bool live = src.at((int) blockIdx.y, w, xj, yj);  // else an id outside the table: the matrix's outputs are zero
+    rows_of_wave<R, RPW>(w, first, [&](auto at_once, auto bytes, int r0) {
+        constexpr int RR = decltype(at_once)::value;
+        float acc[RR][1] = {};
+        if (live) {
+            const tsx_block_q8_1* xs[1] = {xj};
+            const uint8_t* wr[RR];
 #pragma unroll
-        for (int j = 0; j < R; ++j) wr[j] = w + (uint64_t) min(r0 + RPW * j, n_out - 1) * row_bytes;
-        row_dots<T, LPR, 1, R>(wr, xs, 1, n_in / 32, l, tab, acc);
-    }
-    if (l == 0)
+            for (int j = 0; j < RR; ++j) wr[j] = w + (uint64_t) min(r0 + RPW * j, n_out - 1) * row_bytes;
+            row_dots<T, LPR, 1, RR, decltype(bytes)::value>(wr, xs, 1, n_in / 32, l, tab, acc);
+        }
+        if (l == 0)
 #pragma unroll
-        for (int j = 0; j < R; ++j)
-            if (r0 + RPW * j < n_out) yj[r0 + RPW * j] = acc[j][0];
+            for (int j = 0; j < RR; ++j)
+                if (r0 + RPW * j < n_out) yj[r0 + RPW * j] = acc[j][0];
+    });
 }
 
 // the integer contract, one thread per (row, unit).  Two decoders read units, one from global memory (this file's products,
@@ -313,7 +337,7 @@ __global__ void __launch_bounds__(kThreads) subblock_sums_kernel(const uint8_t* 
             if (i < n_rows * nu) unit_load<T>(s_w, (int) threadIdx.x, wu, grid_const());
         }
     } else {
-        unit_load_global<T>(w + (uint64_t) r * row_bytes, u, wu, grid_const());
+        unit_load_global<T, true>(w + (uint64_t) r * row_bytes, u, wu, grid_const());
     }
     if (i >= n_rows * nu) return;
     for (int64_t c = 0; c < ncols; ++c) {

@@ -302,18 +302,18 @@ __device__ __forceinline__ void unit_load(const uint8_t* row, int u, Unit& o, co
 // ------------------------------------------------------------------ unit decode from global memory
 // The fields of a unit in global memory, which two-byte loads serve badly (22 of them for a Q4_K unit): the aligned 4-byte
 // words around the fields are read in 16-byte pieces and shifted into place: three load instructions for a Q4_K unit, three
-// for Q8_0, eight for Q6_K.  Only words that hold bytes of the field are read.  A GGUF matrix starts on a 4-byte boundary
-// and its rows on 2-byte ones; any other byte address (a byte stride of experts, an offset of the caller's) costs the same
-// shifts.  Four dense products of 2048 x 6144 by four columns with their quantize launches: Q6_K 55 -> 41 us, Q8_0 54 ->
-// 40, Q4_K 46 -> 36; IQ3_S, its codebook in LDS (LdsTab), 51 -> 39.
+// for Q8_0, eight for Q6_K.  Only words that hold bytes of the field are read.  BYTES: the row may start on any byte address
+// (a byte stride of experts, an offset of the caller's) instead of a 2-byte one.  Four dense products of 2048 x 6144 by four
+// columns with their quantize launches: Q6_K 55 -> 41 us, Q8_0 54 -> 40, Q4_K 46 -> 36; IQ3_S, its codebook in LDS (LdsTab),
+// 51 -> 39.
 typedef int v4i_a4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef int v2i_a4 __attribute__((ext_vector_type(2), aligned(4)));
 __device__ __forceinline__ uint32_t gld16(uintptr_t a) { return *(gbl_ptr<const uint16_t>) a; }
 __device__ __forceinline__ uint32_t gld8(uintptr_t a) { return *(gbl_ptr<const uint8_t>) a; }
-// 4 N bytes at a (any byte address) as N words, N = 1, 2, 4 or 8
-template <int N> __device__ __forceinline__ void gld_words(uintptr_t a, uint32_t (&w)[N]) {
+// 4 N bytes at a as N words, N = 1, 2, 4 or 8; BYTES: a any byte address, else on a 2-byte boundary
+template <int N, bool BYTES> __device__ __forceinline__ void gld_words(uintptr_t a, uint32_t (&w)[N]) {
     const uintptr_t b = a & ~(uintptr_t) 3;
-    const uint32_t off = (uint32_t) a & 3u, sh = 8 * off;
+    const uint32_t sh = BYTES ? (uint32_t) (a & 3) * 8 : (uint32_t) (a & 2) * 8;
     uint32_t r[N + 1];
     if constexpr (N >= 4) {
 #pragma unroll
@@ -330,11 +330,11 @@ template <int N> __device__ __forceinline__ void gld_words(uintptr_t a, uint32_t
         r[0] = *(gbl_ptr<const uint32_t>) b;
     }
     // the word after: read where the bytes straddle, else the last one again
-    r[N] = *(gbl_ptr<const uint32_t>) (b + 4 * (N - 1) + ((off + 3u) & 4u));
+    r[N] = *(gbl_ptr<const uint32_t>) (b + 4 * (N - 1) + (BYTES ? ((a & 3) + 3) & 4 : 2 * (a & 2)));
 #pragma unroll
     for (int k = 0; k < N; ++k) w[k] = __builtin_amdgcn_alignbit(r[k + 1], r[k], sh);
 }
-template <int T, typename Tab>
+template <int T, bool BYTES = false, typename Tab>
 __device__ __forceinline__ void unit_load_global(const uint8_t* row, int u, Unit& o, const Tab& g) {
     const uintptr_t blk = (uintptr_t) row + (uintptr_t) (u / Fmt<T>::upb * Fmt<T>::bytes);
     const int j = u % Fmt<T>::upb;
@@ -342,8 +342,8 @@ __device__ __forceinline__ void unit_load_global(const uint8_t* row, int u, Unit
     if constexpr (T == TSX_IQ3_XXS) {
         uint32_t q[2], aux[1];
         const float d = h2f((uint16_t) gld16(blk));
-        gld_words<2>(blk + 2 + 8 * j, q);
-        gld_words<1>(blk + 66 + 4 * j, aux);
+        gld_words<2, BYTES>(blk + 2 + 8 * j, q);
+        gld_words<1, BYTES>(blk + 66 + 4 * j, aux);
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
             const SignEntry sg = tab_sign<TSX_IQ3_XXS>(g, (aux[0] >> (7 * l)) & 127u);
@@ -355,8 +355,8 @@ __device__ __forceinline__ void unit_load_global(const uint8_t* row, int u, Unit
     } else if constexpr (T == TSX_IQ3_S) {
         uint32_t q[2], sb[1];
         const float d = h2f((uint16_t) gld16(blk));
-        gld_words<2>(blk + 2 + 8 * j, q);
-        gld_words<1>(blk + 74 + 4 * j, sb);
+        gld_words<2, BYTES>(blk + 2 + 8 * j, q);
+        gld_words<1, BYTES>(blk + 74 + 4 * j, sb);
         const uint32_t qh = gld8(blk + 66 + j);
         const uint32_t sc = (gld8(blk + 106 + (j >> 1)) >> (4 * (j & 1))) & 15u;
 #pragma unroll
@@ -371,8 +371,8 @@ __device__ __forceinline__ void unit_load_global(const uint8_t* row, int u, Unit
         o.a = d * (float) (2 * (int) sc + 1);
     } else if constexpr (T == TSX_Q4_K) {
         uint32_t h[4], q[8];
-        gld_words<4>(blk, h);
-        gld_words<8>(blk + 16 + 32 * (j >> 1), q);
+        gld_words<4, BYTES>(blk, h);
+        gld_words<8, BYTES>(blk + 16 + 32 * (j >> 1), q);
         const int sh = 4 * (j & 1);
 #pragma unroll
         for (int k = 0; k < 8; ++k) o.w[k] = (int) ((q[k] >> sh) & 0x0F0F0F0Fu);
@@ -380,7 +380,7 @@ __device__ __forceinline__ void unit_load_global(const uint8_t* row, int u, Unit
     } else if constexpr (T == TSX_Q4_0) {
         // the 4-bit codes as they are (0..15); the -8 offset is applied with the activation block's sum
         uint32_t q[4];
-        gld_words<4>(blk + 2, q);
+        gld_words<4, BYTES>(blk + 2, q);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {  // values 4 k .. 4 k + 3, and 16 + 4 k ..
             o.w[k] = (int) (q[k] & 0x0F0F0F0Fu);
@@ -394,8 +394,8 @@ __device__ __forceinline__ void unit_load_global(const uint8_t* row, int u, Unit
         // unsigned (0..63): the -32 is applied with each half's activation sum
         const int half = j >> 2, qt = j & 3, lsh = 4 * (qt >> 1), hsh = 2 * qt;
         uint32_t ql[8], qh[8];
-        gld_words<8>(blk + 64 * half + 32 * (qt & 1), ql);
-        gld_words<8>(blk + 128 + 32 * half, qh);
+        gld_words<8, BYTES>(blk + 64 * half + 32 * (qt & 1), ql);
+        gld_words<8, BYTES>(blk + 128 + 32 * half, qh);
 #pragma unroll
         for (int k = 0; k < 8; ++k)
             o.w[k] = (int) (((ql[k] >> lsh) & 0x0F0F0F0Fu) | (((qh[k] >> hsh) & 0x03030303u) << 4));
@@ -405,7 +405,7 @@ __device__ __forceinline__ void unit_load_global(const uint8_t* row, int u, Unit
         o.a = h2f((uint16_t) gld16(blk + 208));
     } else {
         uint32_t q[8];
-        gld_words<8>(blk + 2, q);
+        gld_words<8, BYTES>(blk + 2, q);
 #pragma unroll
         for (int k = 0; k < 8; ++k) o.w[k] = (int) q[k];
         o.a = h2f((uint16_t) gld16(blk));

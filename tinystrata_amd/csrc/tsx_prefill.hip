@@ -141,9 +141,10 @@ __global__ void __launch_bounds__(kThreads) mmq_quantize1_kernel(const float* __
 }
 
 // ------------------------------------------------------------------ grouped product (row-dot form)
-// block (row chunk, expert): weight rows of one expert against all of its token rows, kNC tokens per pass
+// block (row chunk, expert): weight rows of one expert against all of its token rows, kNC tokens per pass.  BYTES: some
+// matrix may start on an odd address
 constexpr int kNC = 4;
-template <int T, int LPR>
+template <int T, int LPR, bool BYTES>
 __global__ void __launch_bounds__(kThreads) mmq_rows_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes,
                                                             uint64_t row_bytes, int w_rows, int w_cols, MmqPlanes P,
                                                             const int32_t* __restrict__ bounds,
@@ -166,7 +167,7 @@ __global__ void __launch_bounds__(kThreads) mmq_rows_kernel(const uint8_t* __res
         float acc[kNC] = {0.f, 0.f, 0.f, 0.f};
         for (int u = l; u < nu; u += LPR) {
             Unit wu;
-            unit_load_global<T>(wr, u, wu, tab);
+            unit_load_global<T, BYTES>(wr, u, wu, tab);
 #pragma unroll
             for (int c = 0; c < kNC; ++c) {
                 if (c < n) {
@@ -1730,15 +1731,18 @@ TSX_API int tsx_moe_mmq_run(const tsx_mmq_product* p, void* stream) {
         });
     }
     const int lpr = lanes_per_row((int) (p->w_cols / 32)), rows = (kThreads / kWave) * (kWave / lpr);
-    return with_type(p->type, [&](auto T) {
-        return with_lpr(lpr, [&](auto LPR) {
-            const dim3 grid((unsigned) ((p->w_rows + rows - 1) / rows), (unsigned) p->n);
-            mmq_rows_kernel<decltype(T)::value, decltype(LPR)::value><<<grid, kThreads, 0, s>>>(
-                (const uint8_t*) p->w, p->expert_bytes, rb, (int) p->w_rows, (int) p->w_cols, P, p->bounds, p->ids, p->dst,
-                p->ld_dst);
-            return launch_status("tsx_moe_mmq_run");
+    const auto row_dots = [&](auto bytes) {
+        return with_type(p->type, [&](auto T) {
+            return with_lpr(lpr, [&](auto LPR) {
+                const dim3 grid((unsigned) ((p->w_rows + rows - 1) / rows), (unsigned) p->n);
+                mmq_rows_kernel<decltype(T)::value, decltype(LPR)::value, decltype(bytes)::value><<<grid, kThreads, 0, s>>>(
+                    (const uint8_t*) p->w, p->expert_bytes, rb, (int) p->w_rows, (int) p->w_cols, P, p->bounds, p->ids,
+                    p->dst, p->ld_dst);
+                return launch_status("tsx_moe_mmq_run");
+            });
         });
-    });
+    };
+    return aligned(p->w, 2) && p->expert_bytes % 2 == 0 ? row_dots(std::false_type{}) : row_dots(std::true_type{});
 }
 
 TSX_API int tsx_moe_mmq_gate_up_swiglu(const void* w, int type, int64_t n_ff, int64_t n_embd, uint64_t expert_bytes,
