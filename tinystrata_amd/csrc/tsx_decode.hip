@@ -121,7 +121,7 @@ __global__ void __launch_bounds__(kThreads) expert_gu_kernel(const uint64_t* __r
                                                              const int32_t* __restrict__ ent_tok,
                                                              const tsx_block_q8_1* __restrict__ xq, tsx_expert_layout L,
                                                              float* __restrict__ gate, float* __restrict__ up) {
-    __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
+    __shared__ __attribute__((aligned(8))) uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
     const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
     if constexpr (lds_tab_words<T>() > 0) __syncthreads();
     constexpr int RPW = kWave / LPR;
@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(kThreads) expert_down_kernel(const uint64_t* _
                                                                const int32_t* __restrict__ ent_dst,
                                                                const tsx_block_q8_1* __restrict__ hq, tsx_expert_layout L,
                                                                float* __restrict__ out) {
-    __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
+    __shared__ __attribute__((aligned(8))) uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
     const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
     if constexpr (lds_tab_words<T>() > 0) __syncthreads();
     constexpr int RPW = kWave / LPR;
@@ -213,7 +213,7 @@ template <int T, int LPR, int R>
 __global__ void __launch_bounds__(kThreads) mmvq_kernel(const uint8_t* __restrict__ w, uint64_t row_bytes,
                                                         const tsx_block_q8_1* __restrict__ x, float* __restrict__ y,
                                                         int n_in, int n_out, int ncols) {
-    __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
+    __shared__ __attribute__((aligned(8))) uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
     const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
     if constexpr (lds_tab_words<T>() > 0) __syncthreads();
     constexpr int RPW = kWave / LPR;
@@ -278,7 +278,7 @@ struct SlotsSource {
 };
 template <int T, int LPR, int R, typename Src>
 __global__ void __launch_bounds__(kThreads) mmvq_many_kernel(Src src, uint64_t row_bytes, int n_in, int n_out) {
-    __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
+    __shared__ __attribute__((aligned(8))) uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
     const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
     if constexpr (lds_tab_words<T>() > 0) __syncthreads();
     constexpr int RPW = kWave / LPR;

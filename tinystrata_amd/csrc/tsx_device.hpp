@@ -157,18 +157,32 @@ template <int T>
 struct LdsTab {
     lds_ptr<const uint32_t> grid, sign;
 };
-// every thread of the block stores its share; a barrier has to follow before the first read
+// the words this thread stores, all requested together (lds_tab_fetch), and their stores (a barrier has to follow before the
+// first read)
+template <int T, int NT> struct LdsTabWords {
+    static constexpr int NG = rep_grid_entries<T>(), N = lds_tab_words<T>(), PER = N / NT;
+    static_assert(NG % NT == 0 && N % NT == 0, "whole rounds of the block's threads");
+    uint32_t v[PER > 0 ? PER : 1];
+};
 template <int T, int NT>
-__device__ __forceinline__ LdsTab<T> lds_tab_fill(uint32_t* lds) {
-    constexpr int NG = rep_grid_entries<T>(), N = lds_tab_words<T>();
+__device__ __forceinline__ void lds_tab_fetch(LdsTabWords<T, NT>& w) {
     const uint32_t* g = T == TSX_IQ3_XXS ? kGrid.xxs : kGrid.s;
     const uint32_t* sg = (const uint32_t*) (T == TSX_IQ3_XXS ? kGrid.xxs_sign : kGrid.s_sign);
+    const int tid = (int) threadIdx.x;
 #pragma unroll
-    for (int k = 0; k < (N + NT - 1) / NT; ++k) {
-        const int i = (int) threadIdx.x + NT * k;
-        if (i < N) ((lds_ptr<uint32_t>) lds)[i] = i < NG ? g[i] : sg[i - NG];
-    }
-    return LdsTab<T>{(lds_ptr<const uint32_t>) lds, (lds_ptr<const uint32_t>) lds + NG};
+    for (int k = 0; k < w.PER; ++k) w.v[k] = NT * k < w.NG ? g[tid + NT * k] : sg[tid + NT * k - w.NG];
+}
+template <int T, int NT>
+__device__ __forceinline__ LdsTab<T> lds_tab_store(const LdsTabWords<T, NT>& w, uint32_t* lds) {
+#pragma unroll
+    for (int k = 0; k < w.PER; ++k) ((lds_ptr<uint32_t>) lds)[(int) threadIdx.x + NT * k] = w.v[k];
+    return LdsTab<T>{(lds_ptr<const uint32_t>) lds, (lds_ptr<const uint32_t>) lds + w.NG};
+}
+template <int T, int NT>
+__device__ __forceinline__ LdsTab<T> lds_tab_fill(uint32_t* lds) {
+    LdsTabWords<T, NT> w;
+    lds_tab_fetch(w);
+    return lds_tab_store(w, lds);
 }
 template <int T> __device__ __forceinline__ uint32_t tab_grid(const LdsTab<T>& r, uint32_t i) { return r.grid[i]; }
 template <int T> __device__ __forceinline__ SignEntry tab_sign(const LdsTab<T>& r, uint32_t i) {

@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(kThreads) mmq_rows_kernel(const uint8_t* __res
                                                             const int32_t* __restrict__ bounds,
                                                             const int32_t* __restrict__ ids, float* __restrict__ dst,
                                                             int64_t ld_dst) {
-    __shared__ uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
+    __shared__ __attribute__((aligned(8))) uint32_t s_tab[lds_tab_words<T>() > 0 ? lds_tab_words<T>() : 1];
     const LdsTab<T> tab = lds_tab_fill<T, kThreads>(s_tab);
     if constexpr (lds_tab_words<T>() > 0) __syncthreads();
     constexpr int RPW = kWave / LPR;
