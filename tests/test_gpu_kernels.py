@@ -393,6 +393,38 @@ def test_expert_grouped_grid_groups_invariant():
     assert (outs[0] == outs[1]).all() and (outs[0] == outs[2]).all()
 
 
+@pytest.mark.parametrize("gu,d", [(IQ3_XXS, IQ3_S), (IQ3_S, IQ3_XXS), (Q4_K, Q4_K), (Q8_0, Q8_0)])
+@pytest.mark.parametrize("FF", [256, 768])
+def test_expert_grouped_rows_per_wave(gu, d, FF):
+    """1 to 16 groups in use in a table for 16, under every number of launched block rows: one, two or four rows per wave
+    and lane group, a block with one item or several.  The same bits whatever the launch, against the oracle; the gate/up
+    rows of n_ff 256 and 768 end in half a block's rows."""
+    N, E, n_ent = 2048, 16, 20
+    L, blobs, _ = experts(gu, d, N, FF, E, distinct=5)
+    Lo = O.layout(gu, d, N, FF)
+    rng = np.random.default_rng(FF + gu)
+    xq = O.quantize_q8_1(rng.normal(0, 1, (n_ent, N)).astype(np.float32))
+    blobs_d, xq_d = dev(blobs.ravel()), dev(xq)
+    for live in (1, 4, 5, 9, 16):
+        ids = np.sort(np.arange(n_ent) % live).astype(np.int32).reshape(n_ent, 1)
+        _, egs, g, eed, eet = O.group(ids, 1, E)
+        assert g == live
+        exp = O.expert_down(Lo, [blobs[x] for x in range(live)], egs, eed,
+                            O.expert_gu(Lo, [blobs[x] for x in range(live)], egs, eet, xq)[1], n_ent)
+        gp, gs, ng, ed, et = ops.group_entries(dev(ids), 1, E, blobs_d.data_ptr(), blobs.shape[1])
+        first = None
+        for gg in (1, 0, 4, 8, 11):
+            print(f"grouped rows per wave gu={gu} FF={FF} live={live} grid_groups={gg}", flush=True)
+            scratch = torch.zeros(ops.native_expert_scratch_bytes(n_ent, FF), dtype=torch.uint8, device="cuda")
+            out = torch.full((n_ent, N), float("nan"), device="cuda")
+            ops.native_expert_grouped(L, gp, gs, ng, ed, et, E, n_ent, xq_d, scratch, out, grid_groups=gg)
+            got = host(out)
+            if first is None:
+                first = got
+                assert rel_l2(got, exp) < 1e-3
+            assert np.array_equal(got, first)
+
+
 # ------------------------------------------------------------------ grouped prompt products
 @pytest.mark.parametrize("t", TYPES)
 @pytest.mark.parametrize("w_cols", [256, 512, 2048])
