@@ -537,6 +537,33 @@ def test_mmq_run_few_rows(t, w_cols, w_rows, pad):
     assert (np.abs(got[:, :w_rows] - exp) <= 1e-5 * np.abs(exp) + 1e-5 * scale).all()
 
 
+@pytest.mark.parametrize("t", TYPES)
+@pytest.mark.parametrize("n,rows,w_rows", [(1, 16, 192), (1, 64, 2112), (64, 16, 2048), (64, 512, 2048), (64, 64, 2112)])
+def test_mmq_run_few_rows_passes(t, n, rows, w_rows):
+    """A short row's one and two passes over the output columns, by the tiles that the bounds give: few tiles of one expert,
+    all rows on two of 64 experts, and every expert with a row or eight; column counts that end in half a block of one pass
+    and of two.  Every output, against the oracle."""
+    rng = np.random.default_rng(t + n + rows)
+    cols, kinds = 256, min(n, 3)
+    W = [ops.quantize_weights(t, rng.normal(0, 0.02, (w_rows, cols)).astype(np.float32)) for _ in range(kinds)]
+    eb = (W[0].size + 255) // 256 * 256
+    blob = np.zeros((kinds, eb), np.uint8)
+    for i, m in enumerate(W):
+        blob[i, :m.size] = m.ravel()
+    blob_d = dev(blob)[torch.arange(n, device="cuda") % kinds].contiguous()
+    x = rng.normal(0, 1, (rows, cols)).astype(np.float32)
+    xb = O.quantize_q8_1(x)
+    each = [O.mmvq_q8_1(t, m, cols, w_rows, xb, rows) for m in W]
+    xq = ops.mmq_quantize(dev(x), None, t, cols, cols, rows)
+    even, skewed = np.arange(n + 1) * rows // n, np.clip(np.arange(n + 1) - n // 2, 0, 2) * rows // 2
+    for bounds in (even, skewed) if n > 1 else (even,):
+        dst = torch.full((rows, w_rows), float("nan"), device="cuda")
+        ops.mmq_run(blob_d.view(-1), t, w_rows, cols, eb, n, xq, dev(bounds.astype(np.int32)), None, rows, dst, w_rows)
+        owner = np.searchsorted(bounds, np.arange(rows), side="right") - 1
+        exp = np.stack([each[o % kinds][r] for r, o in enumerate(owner)])
+        np.testing.assert_allclose(host(dst), exp, rtol=1e-5, atol=1e-5 * np.abs(exp).max())
+
+
 def _cancelling_pair(t, w, cols):
     """Two places of the first row's first unit whose weights have the same magnitude (Q4_K: the same code), and the sign
     that makes w[i] - sign * w[j] zero: an activation unit (a at i, -sign a at j) whose dot product with the row is 0."""

@@ -1074,6 +1074,11 @@ constexpr int kSUnitRow = 40;                // Q8_0: floats from unit to unit o
 // three for Q4_K, whose raw rows are wider (at four it spills: a batch of 32, gate/up and down 126 -> 117 us a layer with
 // three)
 template <int T> constexpr int small_wpe() { return T == TSX_Q8_0 ? 2 : T == TSX_Q4_K ? 3 : 4; }
+// the blocks of two passes from which a short row (a down product) takes two passes, sharing a block's set-up and
+// activations: with fewer, the blocks of one pass are all on the chip at once (small_wpe of them on each of 256 CUs) and
+// take less time than two passes in a row (one expert of 2048 x 512, 16 rows: Q4_K 10.6 -> 7.0 us, IQ3_XXS 13.5 -> 8.6;
+// more tiles than that: 60 tokens on 128 experts, Q8_0, 44 us with one pass, 39 with two)
+template <int T> constexpr int two_pass_blocks() { return 128 * small_wpe<T>(); }
 template <int T> constexpr int small_grid() { return T == TSX_IQ3_XXS ? 256 : T == TSX_IQ3_S ? 512 : 0; }
 // the codebook (four fp16 magnitudes an entry) and the sixteen masks of four sign bits
 template <int T> constexpr int small_tab_bytes() { return small_grid<T>() > 0 ? 8 * small_grid<T>() + 128 : 0; }
@@ -1203,7 +1208,7 @@ __global__ void __launch_bounds__(64 * kSWaves) __attribute__((amdgpu_waves_per_
 mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t row_bytes, int w_rows, int w_cols,
                  int n_exp, MmqPlanes P, const int32_t* __restrict__ bounds, const int32_t* __restrict__ ids,
                  float* __restrict__ dst, int64_t ld_dst, const int32_t* __restrict__ xids, MmqPlanes H, int nbx,
-                 int passes, int vec4) {
+                 int max_passes, int vec4) {
     using L = SmallLds<T>;
     constexpr int NW = kSWaves, NT = 64 * NW, EPT = kMaxExpertsMmq / NT;
     constexpr int BH = FUSE ? 16 * NW : 32 * NW;  // output columns per block and pass
@@ -1220,7 +1225,6 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
 
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int bx = (int) blockIdx.x % nbx;
     if (tid == 0) s_item[3] = 0;
 
     // the codebook: this thread's grid entries, stored below
@@ -1246,6 +1250,16 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
     }
     uint64_t total;
     uint64_t start = block_scan<NT>(mine, s_scan, total);
+    // one or two passes over output columns, by the tiles that there are
+    int passes = 1;
+    if (max_passes > 1) {
+        const int tiles = field(total, 0) + field(total, 1) + field(total, 2) + field(total, 3), half = (nbx + 1) / 2;
+        if ((int64_t) tiles * half >= two_pass_blocks<T>()) {
+            passes = 2;
+            nbx = half;
+        }
+    }
+    const int bx = (int) (blockIdx.x % (unsigned) nbx);
     int cls = 0, want = (int) (blockIdx.x / (unsigned) nbx);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -1568,12 +1582,17 @@ mmq_small_kernel(const uint8_t* __restrict__ w, uint64_t expert_bytes, uint32_t 
     }
 }
 
-// The few-rows form where a product has at most this many rows per expert on average (the routing's skew is not known
-// here): a layer of 256 experts top-8, IQ3, at 256 tokens 188 -> 157 us with Zipf(1.3) routing, at 400 evenly routed
-// tokens (12.5 rows) 309 -> 217 us, but at 300 skewed ones 155 -> 168; Q4_K, 128 experts, Zipf(1.1): 128 tokens 118 -> 116
-// us, 180 tokens 132 -> 139.  Q8_0, 128 experts, evenly routed: 128 tokens 237 -> 199 us, 256 tokens (16 rows) 254 -> 253,
-// 512 tokens 283 -> 364; Zipf(1.3), 256 experts: 256 tokens 158 -> 150 us, 512 tokens (16 rows) 194 -> 225.  A product over one or a few experts takes it up to kFewRows rows: few blocks in flight, which
-// the 16-row tiles make four times as many of
+// The few-rows form where a product has at most this many rows per expert on average; the routing's skew is not known here.
+// Both sides of the line, 128-row (Q4_K, Q8_0: 64-row) tiles -> few rows:
+//   IQ3, 256 experts, a layer: 256 tokens 259 -> 174 us evenly routed, 137 -> 129 with Zipf(1.3); 300 tokens with Zipf(1.3)
+//   155 -> 168, though 400 evenly routed ones (12.5 rows) 309 -> 217
+//   Q4_K, 128 experts, a layer: 128 tokens 168 -> 150 evenly routed, 124 -> 122 with Zipf(1.1); 180 tokens 132 -> 139
+//   Q8_0, 128 experts, a layer: 128 tokens 236 -> 199, 256 tokens (16 rows) 254 -> 253, 512 tokens 283 -> 364; 256 experts
+//   with Zipf(1.3): 256 tokens 158 -> 150, 512 tokens 194 -> 225
+// Up to four rows it is the faster form under every routing measured, down to all tokens on the same experts.  From five to
+// eight, Q4_K is slower where a few experts hold most rows in full tiles (Zipf(2) and beyond, 128 tokens: gate/up 38 -> 49
+// us): 64-row tiles decode their weights once for four times the rows.  A product over one or a few experts takes it up to
+// kFewRows rows: few blocks in flight, which the 16-row tiles make four times as many of
 constexpr int kFewRowsPerExpert = 8, kFewRows = 64;
 inline bool few_rows(int64_t rows, int64_t experts) {
     return rows <= std::max<int64_t>(kFewRowsPerExpert * experts, kFewRows);
@@ -1698,11 +1717,14 @@ TSX_API int tsx_moe_mmq_run(const tsx_mmq_product* p, void* stream) {
             if (p->total_rows == 0) return TSX_OK;
             return with_type(p->type, [&](auto T) {
                 constexpr int TT = decltype(T)::value;
-                // two passes of a short row (a down product) share a block's set-up and activations
-                const int passes = p->w_cols <= 1024 ? 2 : 1, per = 32 * kSWaves * passes;
-                const int nbx = (int) ((p->w_rows + per - 1) / per);
+                const int passes = p->w_cols <= 1024 ? 2 : 1, nbx = (int) ((p->w_rows + 32 * kSWaves - 1) / (32 * kSWaves));
+                // one pass's blocks where the tiles may turn out few, two passes' where every possible tile is there
+                const int64_t tiles = small_tiles(p->total_rows, p->n);
+                const int64_t blocks = passes == 1 ? nbx * tiles
+                                                   : std::max((nbx + 1) / 2 * tiles,
+                                                              std::min<int64_t>(nbx * tiles, 2 * two_pass_blocks<TT>()));
                 mmq_small_kernel<TT, false>
-                    <<<(unsigned) (nbx * small_tiles(p->total_rows, p->n)), 64 * kSWaves, 0, s>>>(
+                    <<<(unsigned) blocks, 64 * kSWaves, 0, s>>>(
                         (const uint8_t*) p->w, p->expert_bytes, (uint32_t) rb, (int) p->w_rows, (int) p->w_cols, p->n, P,
                         p->bounds, p->ids, p->dst, p->ld_dst, nullptr, MmqPlanes{}, nbx, passes,
                         aligned(p->dst, 16) && p->ld_dst % 4 == 0);
