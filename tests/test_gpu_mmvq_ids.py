@@ -151,6 +151,50 @@ def test_mmvq_ids(t, x_every):
         assert np.array_equal(got[j, :n_out], one)
 
 
+def tiled(t, rows, n, seed, distinct=37):
+    """rows x n of type t that repeat `distinct` rows, and the repeating oracle result of a Q8_1 column block."""
+    w = weights(t, distinct, n, seed)
+    rep = np.tile(w, (rows // distinct + 1, 1))[:rows]
+    return rep, lambda xq, ncols: np.tile(O.mmvq_q8_1(t, w, n, distinct, xq, ncols), (1, rows // distinct + 1))[:, :rows]
+
+
+@pytest.mark.parametrize("t", ALL)
+@pytest.mark.parametrize("n_in,n_out,ncols", [(2048, 4097, 5), (2048, 8195, 1), (256, 32771, 8), (256, 65541, 3)])
+def test_mmvq_several_rows_per_lane_group(t, n_in, n_out, ncols):
+    """Every format with two and with four rows of each lane group (from 4096 and 8192 waves), 64 and 8 lanes a row, a last
+    block of few rows, one to eight columns: every output, against the oracle."""
+    print(f"several rows per lane group t={t} {n_out}x{n_in} ncols={ncols}", flush=True)
+    w, oracle = tiled(t, n_out, n_in, n_out + t)
+    xq = O.quantize_q8_1(np.random.default_rng(t).normal(0, 1, (ncols, n_in)).astype(np.float32))
+    exp = oracle(xq, ncols)
+    y = torch.full((ncols * n_out + 8,), 7.0, device="cuda")
+    ops.iq_mmvq(t, dev(w), dev(xq), n_in, n_out, ncols, y=y)
+    got = host(y)
+    assert (got[ncols * n_out:] == 7.0).all()
+    np.testing.assert_allclose(got[:ncols * n_out].reshape(ncols, n_out), exp, rtol=1e-5, atol=1e-5 * np.abs(exp).max())
+
+
+@pytest.mark.parametrize("t", ALL)
+@pytest.mark.parametrize("n_in,n_out,count", [(2048, 1031, 4), (2048, 1031, 8), (256, 4099, 9)])
+def test_mmvq_ids_several_rows_per_lane_group(t, n_in, n_out, count):
+    """The id-indexed product with two and four rows of each lane group: a last block of few rows, ids outside the table
+    among the others (zeros), and outputs apart with a sentinel between them."""
+    print(f"ids, several rows per lane group t={t} {n_out}x{n_in} count={count}", flush=True)
+    mats = [tiled(t, n_out, n_in, 500 + t + m) for m in range(2)]
+    buf = dev(np.concatenate([m[0].ravel() for m in mats]))
+    table = torch.tensor([buf.data_ptr() + m * mats[0][0].size for m in range(2)], dtype=torch.int64, device="cuda")
+    ids = np.array([1, 0, -1, 1, 2, 0, 0, 1, 1][:count], np.int32)
+    xq = O.quantize_q8_1(np.random.default_rng(t).normal(0, 1, (count, n_in)).astype(np.float32))
+    y_stride = n_out + 3
+    y = torch.full((count * y_stride,), 7.0, device="cuda")
+    ops.mmvq_ids(t, table, dev(ids), 0, dev(xq), n_in // 32 * 36, 1, y, y_stride, count, n_in, n_out)
+    got = host(y).reshape(count, y_stride)
+    assert (got[:, n_out:] == 7.0).all()
+    for j, i in enumerate(ids):
+        exp = mats[i][1](xq.reshape(count, -1)[j], 1)[0] if 0 <= i < 2 else np.zeros(n_out)
+        np.testing.assert_allclose(got[j, :n_out], exp, rtol=1e-5, atol=1e-5 * np.abs(exp).max())
+
+
 @pytest.mark.parametrize("t", (IQ3_XXS, Q4_0, Q6_K))
 def test_mmvq_slots(t):
     n_in, n_out, count = 768, 48, 5
