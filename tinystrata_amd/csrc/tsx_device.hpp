@@ -263,15 +263,22 @@ __device__ __forceinline__ void unit_load_iq3s(const uint8_t* row, int u, Unit& 
     o.b = 0.f;
 }
 
-// the float factors of a Q4_K block's sub-block j from its four header words (d and dmin, then 12 scale bytes): the scale
-// and min byte of sub-blocks 0-3 are the low 6 bits of bytes 0-3 and 4-7 of the 12, of 4-7 the nibbles of bytes 8-11 with
-// the top 2 bits of bytes 0-3 and 4-7 above them (selected with masks: no branch on the lane's sub-block)
+// a Q4_K block's scale and min bytes, four sub-blocks' each (low: sub-blocks 0-3, else 4-7), from its 12 scale bytes as three
+// words: those of sub-blocks 0-3 are the low 6 bits of bytes 0-3 and 4-7, of 4-7 the nibbles of bytes 8-11 with the top 2
+// bits of bytes 0-3 and 4-7 above them (selected with masks: no branch on the lane's sub-blocks)
+struct Q4KBytes {
+    uint32_t sc, m;
+};
+__device__ __forceinline__ Q4KBytes q4k_bytes(uint32_t w0, uint32_t w1, uint32_t w2, bool low) {
+    const uint32_t lo = 0u - (uint32_t) low;
+    return Q4KBytes{(w0 & 0x3F3F3F3Fu & lo) | (((w2 & 0x0F0F0F0Fu) | ((w0 >> 2) & 0x30303030u)) & ~lo),
+                    (w1 & 0x3F3F3F3Fu & lo) | ((((w2 >> 4) & 0x0F0F0F0Fu) | ((w1 >> 2) & 0x30303030u)) & ~lo)};
+}
+// the float factors of a block's sub-block j from its four header words (d and dmin, then the scale bytes)
 __device__ __forceinline__ void q4k_scales(uint32_t h0, uint32_t h1, uint32_t h2, uint32_t h3, int j, Unit& o) {
-    const uint32_t lo = 0u - (uint32_t) (j < 4);
-    const uint32_t SC = (h1 & 0x3F3F3F3Fu & lo) | (((h3 & 0x0F0F0F0Fu) | ((h1 >> 2) & 0x30303030u)) & ~lo);
-    const uint32_t M = (h2 & 0x3F3F3F3Fu & lo) | ((((h3 >> 4) & 0x0F0F0F0Fu) | ((h2 >> 2) & 0x30303030u)) & ~lo);
-    o.a = h2f((uint16_t) h0) * (float) ((SC >> (8 * (j & 3))) & 255u);
-    o.b = h2f((uint16_t) (h0 >> 16)) * (float) ((M >> (8 * (j & 3))) & 255u);
+    const Q4KBytes b = q4k_bytes(h1, h2, h3, j < 4);
+    o.a = h2f((uint16_t) h0) * (float) ((b.sc >> (8 * (j & 3))) & 255u);
+    o.b = h2f((uint16_t) (h0 >> 16)) * (float) ((b.m >> (8 * (j & 3))) & 255u);
 }
 // (a Q4_K row in LDS starts on a 16-byte boundary: its rows are whole 16-byte pieces and so are the slabs.  Three 16-byte
 // reads instead of 22 of two bytes: the decode layer at eight tokens, 768 x 2048, 76 -> 68 us, at four 33 -> 30)
@@ -304,7 +311,7 @@ __device__ __forceinline__ void unit_load_q80(const uint8_t* row, int u, Unit& o
     o.b = 0.f;
 }
 
-// unit u of a row of an expert format T in LDS; g: where the codebooks are read (RepTab<T>)
+// unit u of a row of an expert format T in LDS; g: where the codebooks are read (RepTab<T>; GridRef for the formats without)
 template <int T, typename Tab>
 __device__ __forceinline__ void unit_load(const uint8_t* row, int u, Unit& o, const Tab& g) {
     if constexpr (T == TSX_IQ3_XXS) unit_load_iq3xxs(row, u, o, g);

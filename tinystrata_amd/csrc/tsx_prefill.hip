@@ -1141,18 +1141,14 @@ template <int T> __device__ __forceinline__ void raw_scales(const MmqRaw<T>& R, 
     if constexpr (T == TSX_Q4_K) {
         const uint32_t dd = (uint32_t) R.h[0];
         S.d = h2f((uint16_t) dd);
-        // sub-blocks 2 g and 2 g + 1: scale and min bytes (sub-blocks 0-3: the low 6 bits of bytes 0-3 and 4-7; 4-7: the
-        // nibbles of bytes 8-11 with the top 2 bits of bytes 0-3 and 4-7 above them)
-        const uint32_t w0 = (uint32_t) R.h[1], w1 = (uint32_t) R.h[2], w2 = (uint32_t) R.h[3];
-        const uint32_t lo = 0u - (uint32_t) (g < 2);
-        const uint32_t SC = (w0 & 0x3F3F3F3Fu & lo) | (((w2 & 0x0F0F0F0Fu) | ((w0 >> 2) & 0x30303030u)) & ~lo);
-        const uint32_t M = (w1 & 0x3F3F3F3Fu & lo) | ((((w2 >> 4) & 0x0F0F0F0Fu) | ((w1 >> 2) & 0x30303030u)) & ~lo);
+        // sub-blocks 2 g and 2 g + 1
+        const Q4KBytes b = q4k_bytes((uint32_t) R.h[1], (uint32_t) R.h[2], (uint32_t) R.h[3], g < 2);
         const int b0 = 16 * (g & 1);
         const float dmin = -h2f((uint16_t) (dd >> 16));
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-            S.m[k] = hpair((SC >> (b0 + 8 * k)) & 255u);
-            S.mn[k] = dmin * (float) ((M >> (b0 + 8 * k)) & 255u);
+            S.m[k] = hpair((b.sc >> (b0 + 8 * k)) & 255u);
+            S.mn[k] = dmin * (float) ((b.m >> (b0 + 8 * k)) & 255u);
         }
     } else {
         S.a[0] = __builtin_amdgcn_alignbit((uint32_t) R.a.y, (uint32_t) R.a.x, sft);
@@ -1788,9 +1784,8 @@ TSX_API int tsx_moe_mmq_gate_up_swiglu(const void* w, int type, int64_t n_ff, in
     const hipStream_t s = (hipStream_t) stream;
     if (few_rows(n_rows, n_exp))
         return with_type(type, [&](auto T) {
-            constexpr int TT = decltype(T)::value;
             const int nbx = (int) ((n_ff + 16 * kSWaves - 1) / (16 * kSWaves));
-            mmq_small_kernel<TT, true><<<(unsigned) (nbx * small_tiles(n_rows, n_exp)), 64 * kSWaves, 0, s>>>(
+            mmq_small_kernel<decltype(T)::value, true><<<(unsigned) (nbx * small_tiles(n_rows, n_exp)), 64 * kSWaves, 0, s>>>(
                 (const uint8_t*) w, expert_bytes, (uint32_t) rb, (int) n_ff, (int) n_embd, n_exp, P, bounds, nullptr,
                 nullptr, 0, xids, H, nbx, 1, 0);
             return launch_status("tsx_moe_mmq_gate_up_swiglu");
