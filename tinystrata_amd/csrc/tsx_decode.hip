@@ -307,26 +307,32 @@ __global__ void __launch_bounds__(kThreads) mmvq_many_kernel(Src src, uint64_t r
     constexpr int RPW = kWave / LPR;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int slot = lane / LPR, l = lane % LPR;
-    const int first = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
+    const int r0 = (blockIdx.x * (kThreads / kWave) + wave) * RPW * R + slot;
     const uint8_t* w = nullptr;
     const tsx_block_q8_1* xj = nullptr;
     float* yj = nullptr;
-    const bool live = src.at((int) blockIdx.y, w, xj, yj);  // else an id outside the table: the matrix's outputs are zero
-    rows_of_wave<R, RPW>(w, first, [&](auto at_once, auto bytes, int r0) {
-        constexpr int RR = decltype(at_once)::value;
-        float acc[RR][1] = {};
-        if (live) {
-            const tsx_block_q8_1* xs[1] = {xj};
-            const uint8_t* wr[RR];
-#pragma unroll
-            for (int j = 0; j < RR; ++j) wr[j] = w + (uint64_t) min(r0 + RPW * j, n_out - 1) * row_bytes;
-            row_dots<T, LPR, 1, RR, decltype(bytes)::value>(wr, xs, 1, n_in / 32, l, tab, acc);
+    float acc[R][1] = {};
+    if (src.at((int) blockIdx.y, w, xj, yj)) {  // else an id outside the table: the matrix's outputs are zero
+        const tsx_block_q8_1* xs[1] = {xj};
+        if (__builtin_expect((uintptr_t) w & 1, 0)) {  // as rows_of_wave
+#pragma unroll 1
+            for (int j = 0; j < R; ++j) {
+                const uint8_t* const wr[1] = {w + (uint64_t) min(r0 + RPW * j, n_out - 1) * row_bytes};
+                float one[1][1];
+                row_dots<T, LPR, 1, 1, true>(wr, xs, 1, n_in / 32, l, tab, one);
+                if (l == 0 && r0 + RPW * j < n_out) yj[r0 + RPW * j] = one[0][0];
+            }
+            return;
         }
-        if (l == 0)
+        const uint8_t* wr[R];
 #pragma unroll
-            for (int j = 0; j < RR; ++j)
-                if (r0 + RPW * j < n_out) yj[r0 + RPW * j] = acc[j][0];
-    });
+        for (int j = 0; j < R; ++j) wr[j] = w + (uint64_t) min(r0 + RPW * j, n_out - 1) * row_bytes;
+        row_dots<T, LPR, 1, R, false>(wr, xs, 1, n_in / 32, l, tab, acc);
+    }
+    if (l == 0)
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+            if (r0 + RPW * j < n_out) yj[r0 + RPW * j] = acc[j][0];
 }
 
 // the integer contract, one thread per (row, unit).  Two decoders read units, one from global memory (this file's products,
